@@ -497,6 +497,19 @@ int fx_hybrid_gemv_segments_rmsnormed(const void *h, int x_dtype, int n_segments
                                       const float *sparse_rows, const float *const *sparse_columns,
                                       const float *tile_sumsq, int n_tiles, const void *norm_weight, float eps,
                                       void *workspace, size_t workspace_bytes, void *out, int K, void *stream);
+/*
+ * decode_layout (deployment.py:118-121, evaluation.py:59-175): the dense weight
+ * [O, K] of a hybrid layout in weight_dtype (fp32, fp16 or bf16), 16-byte
+ * aligned, bitwise the reference's fp32 arithmetic rounded once.  interleaved
+ * != 0: codes [G, O, 32] and sparse_codes [G, O, 2] hold two bits a column
+ * (base b of column i at bit 2 i + b), else the planes of fx_hybrid_gemv.  *bad
+ * (device-accessible, cleared by the caller) becomes 1 when a scale is not
+ * finite or a group's refinement indices are not ascending in [0, 128); the
+ * weight then holds unspecified values in those groups.
+ */
+int fx_hybrid_restore(const uint8_t *codes, const float *rows, const float *columns, const int16_t *indices,
+                      const uint8_t *sparse_codes, const float *sparse_rows, const float *sparse_columns,
+                      int interleaved, void *weight, int weight_dtype, int *bad, int O, int K, void *stream);
 
 #ifdef __cplusplus
 }

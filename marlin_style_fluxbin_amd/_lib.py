@@ -15,7 +15,7 @@ from pathlib import Path
 import torch
 
 LIBRARY_PATH = Path(__file__).resolve().parent / "libfluxbin_amd.so"
-ABI_VERSION = 19
+ABI_VERSION = 20
 PAYLOAD_PLANAR, PAYLOAD_FIELDS, PAYLOAD_FP6 = 0, 1, 2  # FX_W3_PLANAR / FX_W3_FIELDS / FX_W3_FP6
 
 FX_F32, FX_F16, FX_BF16 = 0, 1, 2
@@ -76,6 +76,7 @@ SIGNATURES: dict[str, tuple] = {
     "fx_hybrid_gemv_residual": (_i, [_p, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _p]),
     "fx_hybrid_gemv_segments_rmsnormed": (_i, [_p, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _f, _p, _sz,
                                                 _p, _i, _p]),
+    "fx_hybrid_restore": (_i, [_p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _p, _i, _i, _p]),
 }
 
 _lock = threading.Lock()

@@ -568,7 +568,7 @@ bool two_base_config(int O, int G, int waves, int prefetch, int groups_per_split
 
 extern "C" {
 
-int fx_abi_version(void) { return 19; }
+int fx_abi_version(void) { return 20; }
 
 const char* fx_last_error(void) { return g_error; }
 
@@ -1602,6 +1602,27 @@ int fx_hybrid_gemv_segments_rmsnormed(const void* h, int x_dtype, int n_segments
   res.pro_eps = eps;
   return run_hybrid(h, x_dtype, n_segments, segment_rows, codes, rows, columns, indices, sparse_codes, sparse_rows,
                     sparse_columns, workspace, workspace_bytes, out, K, res, false, static_cast<hipStream_t>(stream));
+}
+
+int fx_hybrid_restore(const uint8_t* codes, const float* rows, const float* columns, const int16_t* indices,
+                      const uint8_t* sparse_codes, const float* sparse_rows, const float* sparse_columns,
+                      int interleaved, void* weight, int weight_dtype, int* bad, int O, int K, void* stream) {
+  if (!codes || !rows || !columns || !indices || !sparse_codes || !sparse_rows || !sparse_columns || !weight || !bad)
+    return fail(FX_EINVAL, "every layout field, weight and bad must be non-null");
+  if (!is_half_dtype(weight_dtype) && weight_dtype != FX_F32)
+    return fail(FX_EINVAL, "weight dtype must be fp32, fp16 or bf16");
+  if (O < 1 || O > 65536) return fail(FX_EINVAL, "O must be in [1, 65536], got %d", O);
+  if (K < 128 || K > 131072 || K % 128) return fail(FX_EINVAL, "K must be a multiple of 128 in [128, 131072]");
+  if (reinterpret_cast<uintptr_t>(weight) % 16 != 0) return fail(FX_EINVAL, "weight must be 16-byte aligned");
+  const void* vec[3] = {rows, sparse_rows, columns};
+  for (const void* p : vec)
+    if (reinterpret_cast<uintptr_t>(p) % 8 != 0) return fail(FX_EINVAL, "scales must be 8-byte aligned");
+  if (reinterpret_cast<uintptr_t>(codes) % 2 != 0 || reinterpret_cast<uintptr_t>(sparse_codes) % 2 != 0)
+    return fail(FX_EINVAL, "codes must be 2-byte aligned");
+  const fx::HybridRestoreArgs a{codes,          rows,   columns, indices, sparse_codes, sparse_rows,
+                                sparse_columns, weight, bad,     O,       K / 128,      interleaved != 0};
+  fx::launch_hybrid_restore(weight_dtype, a, static_cast<hipStream_t>(stream));
+  return check_launch("hybrid_restore_kernel");
 }
 
 }  // extern "C"

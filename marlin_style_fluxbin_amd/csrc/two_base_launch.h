@@ -89,4 +89,19 @@ enum : int { kHyProPlain = 0, kHyProNorm = 1, kHyProSwiglu = 2 };
 // with every prologue.  False otherwise.
 bool dispatch_hybrid(int xdt, int tiles, int kparts, int prologue, const HybridArgs& a, dim3 grid, hipStream_t s);
 
+// The layout's dense weight (hybrid_restore.hip).
+struct HybridRestoreArgs {
+  const uint8_t* codes;  // [G, O, 2, 16] planes, or [G, O, 32] two bits a column
+  const float* rows;
+  const float* columns;
+  const int16_t* indices;
+  const uint8_t* sparse_codes;
+  const float* sparse_rows;
+  const float* sparse_columns;
+  void* weight;  // [O, 128 G], 16-byte aligned
+  int* bad;
+  int O, G, interleaved;
+};
+void launch_hybrid_restore(int weight_dtype, const HybridRestoreArgs& a, hipStream_t stream);
+
 }  // namespace fx

@@ -34,6 +34,7 @@ from typing import Callable, Mapping
 
 import torch
 from torch import nn
+from torch.nn import functional as F
 
 from . import _lib
 from .evaluation import materialize_hybrid_s8_weight, tensor_sha256
@@ -191,8 +192,66 @@ def restore_artifact(layout: Mapping[str, torch.Tensor]) -> dict[str, torch.Tens
     return payload
 
 
+_RESTORE_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
+
+
+def _restore_kernel_takes(p: Mapping[str, torch.Tensor], dtype) -> bool:
+    """The layouts ``fx_hybrid_restore`` reads: one GPU, contiguous fields of the
+    types and shapes ``convert_artifact`` writes, aligned to their elements' pairs.
+    The torch arithmetic takes (or refuses) every other one."""
+    codes = p["codes"]
+    if not codes.is_cuda or dtype not in _RESTORE_DTYPES or torch.cuda.is_current_stream_capturing():
+        return False
+    g, o = codes.shape[0], codes.shape[1] if codes.ndim > 1 else 0
+    planar = codes.ndim == 4
+    shapes = {"codes": (g, o, 2, 16) if planar else (g, o, 32), "rows": (g, o, 2), "columns": (g, GROUP, 2),
+              "indices": (g, REFINED), "sparse_codes": (g, o, 2, 1) if planar else (g, o, 2),
+              "sparse_rows": (g, o, 2), "sparse_columns": (g, REFINED, 2)}
+    types = {"codes": torch.uint8, "sparse_codes": torch.uint8, "indices": torch.int16}
+    if not (1 <= o <= 65536 and 1 <= g <= 1024):
+        return False
+    return all(p[n].shape == s and p[n].dtype == types.get(n, torch.float32) and p[n].device == codes.device
+               and p[n].is_contiguous() and p[n].data_ptr() % 8 == 0 for n, s in shapes.items())
+
+
+class _Restored:
+    """A dense weight being written by ``fx_hybrid_restore`` on the current stream.
+    ``checked()`` waits for that launch alone (work queued behind it runs on) and
+    says whether the layout was valid: the kernel writes its verdict to pinned host
+    memory."""
+
+    def __init__(self, p, dtype):
+        codes = p["codes"]
+        g, o = codes.shape[:2]
+        device = codes.device
+        self.weight = torch.empty((o, g * GROUP), dtype=dtype, device=device)
+        self._bad = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        _lib.check(_lib.library().fx_hybrid_restore(
+            codes.data_ptr(), p["rows"].data_ptr(), p["columns"].data_ptr(), p["indices"].data_ptr(),
+            p["sparse_codes"].data_ptr(), p["sparse_rows"].data_ptr(), p["sparse_columns"].data_ptr(),
+            int(codes.ndim == 3), self.weight.data_ptr(), _lib.dtype_code(dtype), self._bad.data_ptr(), o,
+            g * GROUP, _lib.stream_handle(device)), "fx_hybrid_restore")
+        self._done = torch.cuda.Event()
+        self._done.record(torch.cuda.current_stream(device))
+
+    def checked(self) -> bool:
+        self._done.synchronize()
+        return int(self._bad[0]) == 0
+
+
 def decode_layout(p: Mapping[str, torch.Tensor], dtype=torch.bfloat16) -> torch.Tensor:
-    """Dense weight ``[O, K]`` of a layout (the dequantize of the dense fallback)."""
+    """Dense weight ``[O, K]`` of a layout (the dequantize of the dense fallback).
+    GPU layouts take ``fx_hybrid_restore``, bitwise the same; one that it finds
+    invalid goes through the torch arithmetic, whose checks name the fault."""
+    if _restore_kernel_takes(p, dtype):
+        with torch.cuda.device(p["codes"].device):
+            restored = _Restored(p, dtype)
+        if restored.checked():
+            return restored.weight
+    return _decode_layout_torch(p, dtype)
+
+
+def _decode_layout_torch(p: Mapping[str, torch.Tensor], dtype) -> torch.Tensor:
     return materialize_hybrid_s8_weight(**restore_artifact(p), group_size=GROUP, columns_per_group=REFINED,
                                         device=p["codes"].device, output_dtype=dtype)
 
@@ -327,6 +386,20 @@ class PackedHybridLinear(PackedLinearBase):
 
     def _dense_weight(self, dtype: torch.dtype) -> torch.Tensor:
         return decode_layout(self.layout(), dtype)
+
+    def _dense_linear(self, x: torch.Tensor) -> torch.Tensor:
+        # the product is queued before the host waits for the layout's verdict
+        layout = self.layout()
+        if _restore_kernel_takes(layout, x.dtype):
+            with torch.cuda.device(layout["codes"].device):
+                restored = _Restored(layout, x.dtype)
+            try:
+                y = F.linear(x, restored.weight, self.bias)
+            finally:
+                valid = restored.checked()
+            if valid:
+                return y
+        return F.linear(x, _decode_layout_torch(layout, x.dtype), self.bias)
 
     def _check_before_call(self) -> None:
         if any(getattr(self, n).dtype != torch.float32 for n in _SCALE_BUFFERS):

@@ -64,6 +64,10 @@ class PackedLinearBase(nn.Module):
         """``[O, K]`` weight of the dense fallback in ``dtype``."""
         raise NotImplementedError
 
+    def _dense_linear(self, x: torch.Tensor) -> torch.Tensor:
+        """The dense fallback's product."""
+        return F.linear(x, self._dense_weight(x.dtype), self.bias)
+
     def _packed_kernel(self, rows: int, device: torch.device) -> PackedKernel:
         """The packed-route callable for ``rows`` activation rows."""
         raise NotImplementedError
@@ -150,7 +154,7 @@ class PackedLinearBase(nn.Module):
             if self.fallback != "dense":
                 raise ValueError("unsupported input; enable explicit dense fallback if needed")
             self._count(DENSE_FALLBACK)
-            return F.linear(x, self._dense_weight(x.dtype), self.bias)
+            return self._dense_linear(x)
         self._count(PACKED_M1 if rows == 1 else PACKED_SMALL_M)
         out = torch.empty((rows, self.out_features), device=x.device, dtype=x.dtype)
         self._packed_kernel(rows, x.device)(x.reshape(rows, self.in_features).contiguous(), out)

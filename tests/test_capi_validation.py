@@ -85,6 +85,7 @@ DEFAULTS = {
     "fx_hybrid_gemv": HYBRID,
     "fx_hybrid_gemv_residual": HYBRID,
 }
+DEFAULTS["fx_hybrid_restore"] = dict(HYBRID, interleaved=0, weight=D, weight_dtype=2, bad=D)
 DEFAULTS["fx_lm_head_logits"] = DEFAULTS["fx_lm_head_argmax"]
 DEFAULTS["fx_decode_attention_rope"] = dict(DEFAULTS["fx_decode_attention"], k=D, v=D, q_norm_weight=D,
                                             k_norm_weight=D, cos=D, sin=D, eps=1e-6, rope_mode=1)
@@ -279,6 +280,13 @@ CASES = [
     ("fx_hybrid_gemv", dict(sparse_rows=None), "non-null"),
     ("fx_hybrid_gemv_residual", dict(residual=None), "residual, out and tile_sumsq must be non-null"),
     ("fx_hybrid_gemv_residual", dict(O=16, K=131072), "the residual epilogue takes one"),
+    ("fx_hybrid_restore", dict(bad=None), "weight and bad must be non-null"),
+    ("fx_hybrid_restore", dict(weight_dtype=5), "weight dtype must be fp32, fp16 or bf16"),
+    ("fx_hybrid_restore", dict(O=65537), "O must be in [1, 65536]"),
+    ("fx_hybrid_restore", dict(K=200), "K must be a multiple of 128 in [128, 131072]"),
+    ("fx_hybrid_restore", dict(weight=D + 8), "weight must be 16-byte aligned"),
+    ("fx_hybrid_restore", dict(rows=D + 4), "scales must be 8-byte aligned"),
+    ("fx_hybrid_restore", dict(codes=D + 1), "codes must be 2-byte aligned"),
 ]
 
 
