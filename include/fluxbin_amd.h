@@ -258,6 +258,19 @@ int fx_w3_gemv_config(const void *x, int x_dtype, const uint8_t *planes, const v
 int fx_w3_restore(const uint8_t *planes, const void *scales, int scale_dtype,
                   const uint8_t *zeros, const int16_t *perm, void *weight, int weight_dtype,
                   int O, int K, void *stream);
+/*
+ * The product of the dense fallback (w3_lut_deployment.py:327-333): out [M, O] =
+ * x [M, K] @ W.T + bias with fx_w3_restore's weight in x_dtype, formed in registers
+ * (no [O, K] weight is written), fp32 accumulation, the bias added in fp32 and one
+ * rounding.  M in [1, 8192].  perm NULL is the identity; entries outside [0, K)
+ * read zero.  bias [O] in x_dtype or NULL.  x, perm and the workspace 16-byte
+ * aligned; the workspace holds the packed activations and, where K is split, the
+ * fp32 partials.  Two launches, three where K is split.
+ */
+size_t fx_w3_gemm_workspace_bytes(int M, int O, int K);
+int fx_w3_gemm(const void *x, int x_dtype, const uint8_t *planes, const void *scales, int scale_dtype,
+               const uint8_t *zeros, const int16_t *perm, const void *bias, void *workspace, size_t workspace_bytes,
+               void *out, int M, int O, int K, void *stream);
 
 /*
  * Reference: rms_norm_reference / fused_rms_norm_forward (fused_modules.py:30-63),

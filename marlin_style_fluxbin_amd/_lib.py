@@ -53,6 +53,8 @@ SIGNATURES: dict[str, tuple] = {
     "fx_w3_gemv_config_workspace_bytes": (_sz, [_i, _i, _i, _i, _i, _i, _i]),
     "fx_w3_gemv_config": (_i, [_p, _i, _p, _p, _i, _p, _p, _p, _sz, _p, _i, _i, _i, _i, _i, _i, _i, _p]),
     "fx_w3_restore": (_i, [_p, _p, _i, _p, _p, _p, _i, _i, _i, _p]),
+    "fx_w3_gemm_workspace_bytes": (_sz, [_i, _i, _i]),
+    "fx_w3_gemm": (_i, [_p, _i, _p, _p, _i, _p, _p, _p, _p, _sz, _p, _i, _i, _i, _p]),
     "fx_rmsnorm": (_i, [_p, _p, _p, _p, _p, _i, _i, _f, _i, _p]),
     "fx_head_norm_rope": (_i, [_i, _p, _p, _p, _p, _p, _p, _i, _i, _i, _p, _p, _p, _p, _f, _i, _i, _p]),
     "fx_decode_attention_workspace_bytes": (_sz, [_i, _i, _i]),

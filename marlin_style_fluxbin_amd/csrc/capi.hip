@@ -16,6 +16,7 @@
 #include "decode_launch.h"
 #include "lm_head_launch.h"
 #include "two_base_launch.h"
+#include "w3_gemm_launch.h"
 
 using fx::LutArgs;
 using fx::MfmaArgs;
@@ -1171,6 +1172,94 @@ int fx_w3_restore(const uint8_t* planes, const void* scales, int scale_dtype,
                      dim3(fx::kRestoreStageThreads), size_t(rows) * K * 2, s, planes, sc, zeros,
                      perm, w, O, G, rows, weight16, perm16);
   return check_launch("w3_restore_permuted_kernel");
+}
+
+namespace {
+
+// Tiling of the W3 GEMM.  The activation tile is the smallest that holds the rows
+// (past 112 rows, 7 or 8 tiles of 16, whichever pads less).  Its wide form (3 or 4
+// output tiles a workgroup: each activation operand feeds that many) runs where it
+// gives three quarters of the CUs a workgroup; else the narrow form, one tile (two
+// with 64 rows and more, or where K is split: twice the rows per operand).  K is
+// split over workgroups only where the grid leaves half of the CUs without one and
+// every wave still has a batch: the splits' fp32 partials cost a finish launch.
+// Measured (bf16, us a launch, 40 rotating payloads in a graph; 37 rows): 12288 x
+// 4096 wide 12.6, two tiles 16.6, one 17.4; 4096 x 4096 one tile 7.0, two tiles in
+// two splits 6.4 + finish; 4096 x 12288 two tiles in two splits 12.0, one tile
+// unsplit 15.8.  512 rows: 4 x 8 tiles 68.4 / 23.7 / 53.5 at the three, 2 x 8 84 / 30 / -.
+fx::GemmPlan gemm_plan(int M, int O, int G) {
+  const int cus = device_cu_count(), batches = (G + 3) / 4, tiles = (O + 15) / 16;
+  fx::GemmPlan p{};
+  if (M <= 64) p.mt = (M + 15) / 16;
+  else p.mt = (M + 111) / 112 * 112 < (M + 127) / 128 * 128 ? 7 : 8;
+  const int row_blocks = (M + 16 * p.mt - 1) / (16 * p.mt);
+  const auto groups = [&](int rt) { return size_t((tiles + rt - 1) / rt) * size_t(row_blocks); };
+  const int wide = p.mt <= 4 ? 3 : 4;
+  if (groups(wide) * 4 >= size_t(cus) * 3) p.rt = wide;
+  else p.rt = p.mt >= 4 || batches >= 16 ? 2 : 1;
+  p.nk = p.mt <= 4 || (p.mt == 7 && p.rt == 2) ? 8 : 4;
+  const size_t n = groups(p.rt);
+  p.splits = 1;
+  if (n * 2 <= size_t(cus)) p.splits = int(std::max<size_t>(1, std::min(size_t(cus) / n, size_t(batches / p.nk))));
+  p.batches_per_split = (batches + p.splits - 1) / p.splits;
+  p.splits = (batches + p.batches_per_split - 1) / p.batches_per_split;
+  return p;
+}
+
+size_t gemm_packed_bytes(int M, int G, const fx::GemmPlan& p) {
+  return size_t((M + 16 * p.mt - 1) / (16 * p.mt)) * p.mt * size_t((G + 3) / 4) * 16384;
+}
+
+}  // namespace
+
+size_t fx_w3_gemm_workspace_bytes(int M, int O, int K) {
+  if (M < 1 || O < 1 || K < 128 || K % 128) return 0;
+  const fx::GemmPlan p = gemm_plan(M, O, K / 128);
+  return gemm_packed_bytes(M, K / 128, p) + (p.splits > 1 ? size_t(p.splits) * M * O * 4 : 0);
+}
+
+int fx_w3_gemm(const void* x, int x_dtype, const uint8_t* planes, const void* scales, int scale_dtype,
+               const uint8_t* zeros, const int16_t* perm, const void* bias, void* workspace, size_t workspace_bytes,
+               void* out, int M, int O, int K, void* stream) {
+  int rc = validate_payload(x, x_dtype, planes, scales, scale_dtype, 1, O, K, FX_ARITH_STRUCTURAL);
+  if (rc) return rc;
+  if (!out) return fail(FX_EINVAL, "out must be non-null");
+  if (M < 1 || M > fx::kGemmMaxRows) return fail(FX_EINVAL, "M must be in [1, %d], got %d", fx::kGemmMaxRows, M);
+  if (perm && K > 32768) return fail(FX_EINVAL, "int16 permutation entries address K <= 32768");
+  const void* vec[3] = {x, perm, workspace};
+  for (const void* p : vec)
+    if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return fail(FX_EINVAL, "x, perm and workspace must be 16-byte aligned");
+  const size_t need = fx_w3_gemm_workspace_bytes(M, O, K);
+  if (!workspace || workspace_bytes < need)
+    return fail(FX_EINVAL, "the GEMM workspace needs %zu bytes, got %zu", need, workspace ? workspace_bytes : size_t(0));
+  const int G = K / 128;
+  const fx::GemmPlan plan = gemm_plan(M, O, G);
+  const size_t packed = gemm_packed_bytes(M, G, plan);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  int rows = 4;  // staged rows of the permuted packing: at most 64 KB of LDS
+  while (rows > 1 && size_t(rows) * K * 2 > 65536) rows >>= 1;
+  fx::launch_gemm_pack({static_cast<const uint16_t*>(x), perm, static_cast<uint4*>(workspace), M, K, plan.mt, rows}, s);
+  rc = check_launch("gemm_pack_kernel");
+  if (rc) return rc;
+  fx::GemmArgs a{};
+  a.packed = static_cast<const uint4*>(workspace);
+  a.planes = planes;
+  a.scales = static_cast<const uint16_t*>(scales);
+  a.zeros = zeros;
+  a.bias = static_cast<const uint16_t*>(bias);
+  a.partial = plan.splits > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + packed) : nullptr;
+  a.out = static_cast<uint16_t*>(out);
+  a.M = M, a.O = O, a.G = G, a.sdt = scale_dtype;
+  a.batches_per_split = plan.batches_per_split;
+  a.vec = O % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
+  const bool wide = plan.mt >= 4, bf = x_dtype == FX_BF16;
+  const bool ran = wide ? (bf ? fx::dispatch_gemm_wide_bf16(plan, a, s) : fx::dispatch_gemm_wide_f16(plan, a, s))
+                        : (bf ? fx::dispatch_gemm_bf16(plan, a, s) : fx::dispatch_gemm_f16(plan, a, s));
+  if (!ran) return fail(FX_EINVAL, "no GEMM kernel for plan (%d, %d, %d)", plan.rt, plan.mt, plan.nk);
+  rc = check_launch("w3_gemm_kernel");
+  if (rc || plan.splits == 1) return rc;
+  fx::launch_gemm_finish(x_dtype, a, plan.splits, s);
+  return check_launch("gemm_finish_kernel");
 }
 
 int fx_rmsnorm(const void* x, const void* residual, const void* weight, void* out,

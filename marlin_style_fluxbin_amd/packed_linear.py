@@ -26,12 +26,23 @@ from typing import Callable
 
 import torch
 from torch import nn
+from torch.autograd import forward_ad
 from torch.nn import functional as F
 
 HALF_DTYPES = (torch.float16, torch.bfloat16)
 PACKED_M1, DENSE_FALLBACK, PACKED_SMALL_M = "packed_m1", "dense_fallback", "packed_small_m"
 
 PackedKernel = Callable[[torch.Tensor, torch.Tensor], torch.Tensor]  # (x [rows, K], out [rows, O]) -> out
+
+
+def plain_call(x: torch.Tensor) -> bool:
+    """True when a kernel called by address computes what a torch op on ``x`` would:
+    a plain tensor, and no tracer, dispatch or function mode, transform (vmap, jvp)
+    or autocast in force that has to see (or would change) the op."""
+    return (type(x) is torch.Tensor and not torch.is_autocast_enabled("cuda")
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and torch._C._functorch.maybe_current_level() is None and forward_ad._current_level < 0
+            and torch._C._get_tracing_state() is None)
 
 
 class PackedLinearBase(nn.Module):

@@ -25,13 +25,14 @@ import torch
 from torch import nn
 
 from . import _lib
-from .packed_linear import PackedLinearBase, replace_linears_atomically
+from .packed_linear import HALF_DTYPES, PackedLinearBase, plain_call, replace_linears_atomically
 from .gptq_deployment import FIELDS, OPTIONAL_FIELDS, restore_planar_w3, validate_planar_w3
 
 ROW_TILES = (256, 512, 1024)
 EXPERIMENTAL_ROW_TILES = ROW_TILES
 ARITHMETIC_MODES = ("structural", "decoded_bf16")
 MAX_PACKED_ROWS = 8
+GEMM_MAX_ROWS = 1024  # dense-fallback rows that fx_w3_gemm multiplies
 QWEN3_ROW_TILE_BY_SHAPE = {
     (4096, 4096): 256,
     (1024, 4096): 512,
@@ -454,6 +455,37 @@ class PackedW3Linear(PackedLinearBase):
 
     def _dense_weight(self, dtype: torch.dtype) -> torch.Tensor:
         return restore_planar_w3(self.layout(), dtype=dtype, perm_identity=self._perm_identity)
+
+    def _gemm_takes(self, x: torch.Tensor) -> bool:
+        """The dense-fallback inputs that ``fx_w3_gemm`` multiplies; the restored
+        weight and ``F.linear`` take (or refuse) every other one."""
+        planes, bias = self.planes, self.bias
+        return (x.is_cuda and x.dtype in HALF_DTYPES and x.device == planes.device and plain_call(x)
+                and 0 < x.numel() <= GEMM_MAX_ROWS * self.in_features
+                and planes.numel() < 2**31 and planes.data_ptr() % 16 == 0 and self.perm.data_ptr() % 16 == 0
+                and (bias is None or (bias.dtype == x.dtype and bias.device == x.device and bias.is_contiguous())))
+
+    def _dense_linear(self, x: torch.Tensor) -> torch.Tensor:
+        if self._gemm_takes(x):
+            rows = x.numel() // self.in_features
+            flat = x.reshape(rows, self.in_features).contiguous()
+            if flat.data_ptr() % 16 == 0:
+                return self._gemm(flat, rows).view(*x.shape[:-1], self.out_features)
+        return super()._dense_linear(x)
+
+    def _gemm(self, x: torch.Tensor, rows: int) -> torch.Tensor:
+        layout = self.layout()
+        validate_planar_w3(layout, check_values=False)
+        lib, o, k = _lib.library(), self.out_features, self.in_features
+        out = torch.empty((rows, o), dtype=x.dtype, device=x.device)
+        nbytes = lib.fx_w3_gemm_workspace_bytes(rows, o, k)
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+        _lib.check(lib.fx_w3_gemm(
+            x.data_ptr(), _lib.dtype_code(x.dtype), self.planes.data_ptr(), self.scales.data_ptr(),
+            _lib.dtype_code(self.scales.dtype), _lib.ptr(layout.get("zeros")),
+            None if self._perm_identity else self.perm.data_ptr(), _lib.ptr(self.bias), workspace.data_ptr(), nbytes,
+            out.data_ptr(), rows, o, k, _lib.stream_handle(x.device)), "fx_w3_gemm")
+        return out
 
     def _check_before_bind(self, device: torch.device) -> None:
         validate_planar_w3(self.layout(), check_values=False)

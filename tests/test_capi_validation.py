@@ -85,6 +85,7 @@ DEFAULTS = {
     "fx_hybrid_gemv": HYBRID,
     "fx_hybrid_gemv_residual": HYBRID,
 }
+DEFAULTS["fx_w3_gemm"] = dict(W3, bias=None, workspace=D, workspace_bytes=1 << 24)
 DEFAULTS["fx_hybrid_restore"] = dict(HYBRID, interleaved=0, weight=D, weight_dtype=2, bad=D)
 DEFAULTS["fx_lm_head_logits"] = DEFAULTS["fx_lm_head_argmax"]
 DEFAULTS["fx_decode_attention_rope"] = dict(DEFAULTS["fx_decode_attention"], k=D, v=D, q_norm_weight=D,
@@ -280,6 +281,15 @@ CASES = [
     ("fx_hybrid_gemv", dict(sparse_rows=None), "non-null"),
     ("fx_hybrid_gemv_residual", dict(residual=None), "residual, out and tile_sumsq must be non-null"),
     ("fx_hybrid_gemv_residual", dict(O=16, K=131072), "the residual epilogue takes one"),
+    ("fx_w3_gemm", dict(M=0), "M must be in [1, 8192]"),
+    ("fx_w3_gemm", dict(M=8193), "M must be in [1, 8192]"),
+    ("fx_w3_gemm", dict(K=200), "multiple of 128"),
+    ("fx_w3_gemm", dict(out=None), "out must be non-null"),
+    ("fx_w3_gemm", dict(x=D + 8), "16-byte aligned"),
+    ("fx_w3_gemm", dict(perm=D + 2), "16-byte aligned"),
+    ("fx_w3_gemm", dict(perm=D, K=32896), "int16 permutation entries"),
+    ("fx_w3_gemm", dict(workspace=None), "the GEMM workspace needs 16384 bytes, got 0"),
+    ("fx_w3_gemm", dict(M=64, workspace_bytes=16384), "the GEMM workspace needs 65536 bytes, got 16384"),
     ("fx_hybrid_restore", dict(bad=None), "weight and bad must be non-null"),
     ("fx_hybrid_restore", dict(weight_dtype=5), "weight dtype must be fp32, fp16 or bf16"),
     ("fx_hybrid_restore", dict(O=65537), "O must be in [1, 65536]"),
