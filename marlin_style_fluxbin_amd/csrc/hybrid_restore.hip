@@ -7,25 +7,31 @@
 // arithmetic; contraction to fused multiply-adds would move its last bit.
 //
 // Bound by the store of 2 O K bytes.  A workgroup owns 128 columns (one group) of
-// kHyRestoreRows rows: lane c of a row's 16 lanes expands byte c of the two sign
-// rows into 8 columns and stores them as 16 bytes, so a row's 256 bytes leave
-// together; the group's column scales and the refinement column of each of the
-// lane's 8 columns stay in registers over the rows.  Layout data that the torch
+// kHyRestoreRows rows, a wave eight rows at a time: lane c of a row's 16 lanes expands
+// byte c of the two sign rows into 8 columns, with the group's column scales kept in
+// registers over the rows, and leaves them in the wave's LDS rows; then each of the 64
+// lanes forms one refined column (8 rows x 8 columns, their scales in registers too)
+// and writes it over, and the rows leave as 16-byte stores, 256 bytes of a row
+// together.  (Selecting the refined columns within each lane's eight instead cost more
+// than the rest of the kernel: they are one in sixteen.)  Layout data that the torch
 // arithmetic refuses (a scale that is not finite, refinement columns outside the
 // group or not ascending) sets *bad; such columns are not written through.
 //
 // Measured: the fallback of a Qwen3-8B layer's seven Linears on 200 rows took
 // 13.8 ms with the torch arithmetic (about thirty passes over fp32 and int8
-// [O, K] tensors and four host synchronisations each) and takes 0.52 ms with this
-// kernel and one wait.
+// [O, K] tensors and four host synchronisations each) and takes 0.48 ms with this
+// kernel and one wait (12288 x 4096 about 40 us a launch, 4096 x 4096 about 14).
 #include "common.h"
 #include "two_base_launch.h"
+
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
 namespace fx {
 
-constexpr int kHyRestoreRows = 128;  // rows per workgroup, 16 at a time
+constexpr int kHyRestoreTurns = 2;                     // eight-row turns of a wave, all loaded ahead
+constexpr int kHyRestoreRows = 32 * kHyRestoreTurns;  // rows per workgroup
 
 // The even bits of a 16-bit value, packed (interleaved two-base codes: base b of
 // column i at bit 2 i + b).
@@ -40,14 +46,22 @@ __device__ __forceinline__ float signed_scale(unsigned bit, float v) {  // bit ?
 }
 __device__ __forceinline__ bool not_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
 
+// One weight: (0 + row0 column0) + row1 column1 with the signs' bits (1 = +).
+__device__ __forceinline__ float two_base(unsigned s0, unsigned s1, const float2& row, float c0, float c1) {
+  return (0.f + signed_scale(s0, row.x) * c0) + signed_scale(s1, row.y) * c1;
+}
+
 template <int WDT>
 __global__ __launch_bounds__(256) void hybrid_restore_kernel(HybridRestoreArgs a) {
-  const int c = int(threadIdx.x & 15u), r0 = int(threadIdx.x >> 4);
+  using Element = std::conditional_t<WDT == kF32, float, uint16_t>;
+  constexpr int kVecs = 8 * int(sizeof(Element)) / 16;  // 16-byte vectors of 8 columns
+  __shared__ uint4 stage[4][8][16 * kVecs];
+  const int lane = threadIdx.x & 63, wave = wave_index();
+  const int c = lane & 15;
   const int g = int(blockIdx.x % unsigned(a.G));
   const int o0 = int(blockIdx.x / unsigned(a.G)) * kHyRestoreRows;
   bool bad = false;
-  float col[8][2], ucol[8][2];
-  unsigned slot = 0;  // a nibble per column: refinement slot + 1, or 0
+  float col[8][2];
   {
     const float* cols = a.columns + (size_t(g) * 128 + c * 8) * 2;
 #pragma unroll
@@ -55,76 +69,89 @@ __global__ __launch_bounds__(256) void hybrid_restore_kernel(HybridRestoreArgs a
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         col[e][b] = cols[2 * e + b];
-        ucol[e][b] = 0.f;
         bad |= not_finite(col[e][b]);
       }
     }
-    int previous = -1;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const int idx = a.indices[size_t(g) * 8 + s];
-      const float s0 = a.sparse_columns[(size_t(g) * 8 + s) * 2], s1 = a.sparse_columns[(size_t(g) * 8 + s) * 2 + 1];
-      bad |= idx <= previous || idx > 127 || not_finite(s0) || not_finite(s1);
-      previous = idx;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        if (idx == c * 8 + e) {
-          ucol[e][0] = s0;
-          ucol[e][1] = s1;
-          slot |= unsigned(s + 1) << (4 * e);
-        }
-      }
-    }
   }
-#pragma unroll 2
-  for (int i = r0; i < kHyRestoreRows; i += 16) {
-    const int o = o0 + i;
-    if (o >= a.O) break;
-    const size_t go = size_t(g) * a.O + o;
-    unsigned p0, p1, q0, q1;
-    if (a.interleaved) {
-      const unsigned pair = *reinterpret_cast<const uint16_t*>(a.codes + go * 32 + 2 * c);
-      const unsigned spair = *reinterpret_cast<const uint16_t*>(a.sparse_codes + go * 2);
-      p0 = even_bits(pair), p1 = even_bits(pair >> 1);
-      q0 = even_bits(spair), q1 = even_bits(spair >> 1);
-    } else {
-      p0 = a.codes[go * 32 + c], p1 = a.codes[go * 32 + 16 + c];
-      q0 = a.sparse_codes[go * 2], q1 = a.sparse_codes[go * 2 + 1];
-    }
-    const float2 row = *reinterpret_cast<const float2*>(a.rows + go * 2);
-    const float2 srow = *reinterpret_cast<const float2*>(a.sparse_rows + go * 2);
-    bad |= not_finite(row.x) || not_finite(row.y) || not_finite(srow.x) || not_finite(srow.y);
-    float v[8];
+  // the lane's refined column: slot lane % 8, of rows lane / 8
+  const int slot = lane & 7;
+  const int16_t* indices = a.indices + size_t(g) * 8;
+  const int index = indices[slot];
+  bad |= index < 0 || index > 127 || (slot > 0 && index <= indices[slot > 0 ? slot - 1 : 0]);
+  const int at = index & 127;  // inside the group; a bad index is reported
+  const float2 ucol = *reinterpret_cast<const float2*>(a.sparse_columns + (size_t(g) * 8 + slot) * 2);
+  const float2 rcol = *reinterpret_cast<const float2*>(a.columns + (size_t(g) * 128 + at) * 2);
+  bad |= not_finite(ucol.x) || not_finite(ucol.y);
+  // raw sign bytes of one row: an interleaved pair, or the two planes' bytes
+  const auto signs = [&](const uint8_t* codes, int byte, int width) -> unsigned {
+    if (a.interleaved) return *reinterpret_cast<const uint16_t*>(codes + 2 * byte);
+    return unsigned(codes[byte]) | (unsigned(codes[width + byte]) << 8);
+  };
+  const auto base0 = [&](unsigned v) { return a.interleaved ? even_bits(v) : v & 0xffu; };
+  const auto base1 = [&](unsigned v) { return a.interleaved ? even_bits(v >> 1) : v >> 8; };
+  struct Turn {
+    unsigned codes[2], patch, sparse;  // of the lane's two rows; of its refined column's row
+    float2 row[2], prow, srow;
+  } turn[kHyRestoreTurns];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float t0 = signed_scale((p0 >> e) & 1u, row.x) * col[e][0];
-      const float t1 = signed_scale((p1 >> e) & 1u, row.y) * col[e][1];
-      v[e] = (0.f + t0) + t1;
-    }
-    if (slot) {
+  for (int k = 0; k < kHyRestoreTurns; ++k) {  // rows past O read the last row and are not stored
+    const int i = o0 + wave * 8 * kHyRestoreTurns + 8 * k;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const unsigned s = (slot >> (4 * e)) & 15u;
-        if (s) {
-          const float u0 = signed_scale((q0 >> (s - 1)) & 1u, srow.x) * ucol[e][0];
-          const float u1 = signed_scale((q1 >> (s - 1)) & 1u, srow.y) * ucol[e][1];
-          v[e] = v[e] + ((0.f + u0) + u1);
-        }
+    for (int h = 0; h < 2; ++h) {
+      const size_t go = size_t(g) * a.O + min(i + 4 * h + (lane >> 4), a.O - 1);
+      turn[k].codes[h] = signs(a.codes + go * 32, c, 16);
+      turn[k].row[h] = *reinterpret_cast<const float2*>(a.rows + go * 2);
+    }
+    const size_t go = size_t(g) * a.O + min(i + (lane >> 3), a.O - 1);
+    turn[k].patch = signs(a.codes + go * 32, at >> 3, 16);
+    turn[k].sparse = signs(a.sparse_codes + go * 2, 0, 1);
+    turn[k].prow = *reinterpret_cast<const float2*>(a.rows + go * 2);
+    turn[k].srow = *reinterpret_cast<const float2*>(a.sparse_rows + go * 2);
+  }
+#pragma unroll
+  for (int k = 0; k < kHyRestoreTurns; ++k) {
+    const Turn& in = turn[k];
+    const int i = o0 + wave * 8 * kHyRestoreTurns + 8 * k;
+    if (i >= a.O) break;  // wave-uniform
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const unsigned p0 = base0(in.codes[h]), p1 = base1(in.codes[h]);
+      bad |= not_finite(in.row[h].x) || not_finite(in.row[h].y);
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = two_base((p0 >> e) & 1u, (p1 >> e) & 1u, in.row[h], col[e][0], col[e][1]);
+      uint4* dst = &stage[wave][4 * h + (lane >> 4)][c * kVecs];
+      if constexpr (WDT == kF32) {
+        dst[0] = make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3]));
+        dst[1] = make_uint4(__float_as_uint(v[4]), __float_as_uint(v[5]), __float_as_uint(v[6]), __float_as_uint(v[7]));
+      } else {
+        unsigned pair[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pair[e] = round_pair_bits<WDT>(v[2 * e], v[2 * e + 1]);
+        dst[0] = make_uint4(pair[0], pair[1], pair[2], pair[3]);
       }
     }
-    const size_t at = size_t(o) * (size_t(a.G) * 128) + size_t(g) * 128 + c * 8;
-    if constexpr (WDT == kF32) {
-      float4* dst = reinterpret_cast<float4*>(static_cast<float*>(a.weight) + at);
-      dst[0] = make_float4(v[0], v[1], v[2], v[3]);
-      dst[1] = make_float4(v[4], v[5], v[6], v[7]);
-    } else {
-      uint4 w;
-      unsigned* pair = reinterpret_cast<unsigned*>(&w);
-#pragma unroll
-      for (int e = 0; e < 8; e += 2)
-        pair[e >> 1] = unsigned(from_f32<WDT>(v[e])) | (unsigned(from_f32<WDT>(v[e + 1])) << 16);
-      *reinterpret_cast<uint4*>(static_cast<uint16_t*>(a.weight) + at) = w;
+    {
+      const unsigned p0 = base0(in.patch), p1 = base1(in.patch), q0 = base0(in.sparse), q1 = base1(in.sparse);
+      bad |= not_finite(in.srow.x) || not_finite(in.srow.y);
+      const float w = two_base((p0 >> (at & 7)) & 1u, (p1 >> (at & 7)) & 1u, in.prow, rcol.x, rcol.y) +
+                      two_base((q0 >> slot) & 1u, (q1 >> slot) & 1u, in.srow, ucol.x, ucol.y);
+      __builtin_amdgcn_wave_barrier();  // after the row's own values (LDS operations of a wave run in order)
+      Element* dst = reinterpret_cast<Element*>(&stage[wave][lane >> 3][0]) + at;
+      if constexpr (WDT == kF32) *dst = w;
+      else *dst = from_f32<WDT>(w);
+      __builtin_amdgcn_wave_barrier();
     }
+#pragma unroll
+    for (int n = 0; n < 2 * kVecs; ++n) {
+      const int unit = n * 64 + lane, rr = unit / (16 * kVecs), at16 = unit % (16 * kVecs);
+      const uint4 v = stage[wave][rr][at16];
+      const int o = i + rr;
+      if (o < a.O)
+        *reinterpret_cast<uint4*>(static_cast<Element*>(a.weight) + size_t(o) * (size_t(a.G) * 128) + size_t(g) * 128 +
+                                  at16 * (16 / int(sizeof(Element)))) = v;
+    }
+    __builtin_amdgcn_wave_barrier();
   }
   if (bad) *a.bad = 1;  // every writer stores the same value
 }
