@@ -17,6 +17,7 @@
 #include "lm_head_launch.h"
 #include "two_base_launch.h"
 #include "w3_gemm_launch.h"
+#include "w3_restore_launch.h"
 
 using fx::LutArgs;
 using fx::MfmaArgs;
@@ -1123,23 +1124,6 @@ int fx_w3_gemv_config(const void* x, int x_dtype, const uint8_t* planes, const v
                   static_cast<hipStream_t>(stream));
 }
 
-namespace {
-
-// Kernel pointers of the restore instantiations, indexed [scale bf16][weight bf16].
-using RestoreFn = void (*)(const uint8_t*, const uint16_t*, const uint8_t*, uint16_t*, int, int, int);
-using RestorePermutedFn = void (*)(const uint8_t*, const uint16_t*, const uint8_t*, const int16_t*,
-                                   uint16_t*, int, int, int, int, int);
-constexpr RestoreFn kRestore[2][2] = {
-    {fx::w3_restore_kernel<fx::kF16, fx::kF16>, fx::w3_restore_kernel<fx::kF16, fx::kBF16>},
-    {fx::w3_restore_kernel<fx::kBF16, fx::kF16>, fx::w3_restore_kernel<fx::kBF16, fx::kBF16>}};
-constexpr RestorePermutedFn kRestorePermuted[2][2] = {
-    {fx::w3_restore_permuted_kernel<fx::kF16, fx::kF16>,
-     fx::w3_restore_permuted_kernel<fx::kF16, fx::kBF16>},
-    {fx::w3_restore_permuted_kernel<fx::kBF16, fx::kF16>,
-     fx::w3_restore_permuted_kernel<fx::kBF16, fx::kBF16>}};
-
-}  // namespace
-
 int fx_w3_restore(const uint8_t* planes, const void* scales, int scale_dtype,
                   const uint8_t* zeros, const int16_t* perm, void* weight, int weight_dtype,
                   int O, int K, void* stream) {
@@ -1150,28 +1134,19 @@ int fx_w3_restore(const uint8_t* planes, const void* scales, int scale_dtype,
   if (perm && K > 32768) return fail(FX_EINVAL, "int16 permutation entries address K <= 32768");
   if (reinterpret_cast<uintptr_t>(planes) % 16 != 0)
     return fail(FX_EINVAL, "planes must be 16-byte aligned");
-  const int G = K / 128;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const uint16_t* sc = static_cast<const uint16_t*>(scales);
-  uint16_t* w = static_cast<uint16_t*>(weight);
-  const int sb = scale_dtype == FX_BF16, wb = weight_dtype == FX_BF16;
-  const int weight16 = reinterpret_cast<uintptr_t>(weight) % 16 == 0;
-  if (!perm) {
-    // one workgroup per (16-row block, kRestoreGroups groups)
-    const size_t blocks =
-        size_t((O + 15) / 16) * size_t((G + fx::kRestoreGroups - 1) / fx::kRestoreGroups);
-    if (blocks > size_t(INT32_MAX)) return fail(FX_EINVAL, "O * K too large");
-    hipLaunchKernelGGL(kRestore[sb][wb], dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s,
-                       planes, sc, zeros, w, O, G, weight16);
-    return check_launch("w3_restore_kernel");
-  }
-  // whole rows staged in LDS: at most 32 KB for K <= 16384, one row (<= 64 KB) above
-  const int rows = std::max(1, fx::kRestoreStageBytes / (2 * K));
-  const int perm16 = reinterpret_cast<uintptr_t>(perm) % 16 == 0;
-  hipLaunchKernelGGL(kRestorePermuted[sb][wb], dim3((O + rows - 1) / rows),
-                     dim3(fx::kRestoreStageThreads), size_t(rows) * K * 2, s, planes, sc, zeros,
-                     perm, w, O, G, rows, weight16, perm16);
-  return check_launch("w3_restore_permuted_kernel");
+  const fx::RestoreArgs a{planes,
+                          static_cast<const uint16_t*>(scales),
+                          zeros,
+                          perm,
+                          static_cast<uint16_t*>(weight),
+                          O,
+                          K / 128,
+                          scale_dtype,
+                          reinterpret_cast<uintptr_t>(weight) % 16 == 0,
+                          reinterpret_cast<uintptr_t>(perm) % 16 == 0};
+  if (!fx::launch_restore(weight_dtype, a, static_cast<hipStream_t>(stream)))
+    return fail(FX_EINVAL, "O * K too large");
+  return check_launch("w3_restore_kernel");
 }
 
 namespace {
@@ -1201,6 +1176,25 @@ fx::GemmPlan gemm_plan(int M, int O, int G) {
   const size_t n = groups(p.rt);
   p.splits = 1;
   if (n * 2 <= size_t(cus)) p.splits = int(std::max<size_t>(1, std::min(size_t(cus) / n, size_t(batches / p.nk))));
+  if (M > 128) {
+    // The kernel for many rows works on 192 x 128 outputs at a time, this one on 16 rt x
+    // 16 mt; times per round of workgroups over the CUs from the measurements beside the
+    // kernels (us; per 4096 columns of K), a split's partials at 5 TB/s and its launch.
+    const double k4 = G / 32.0;
+    const auto cost = [&](size_t workgroups, int splits, double start, double per_k) {
+      return double((workgroups * splits + cus - 1) / cus) * (start + per_k * k4 / splits) +
+             (splits > 1 ? 4 + M * 1.6e-6 * O * splits : 0);
+    };
+    double best = cost(n, p.splits, 8, 0.48 * p.rt * p.mt);
+    const size_t tall = size_t((tiles + 11) / 12) * size_t((M + 127) / 128);
+    for (int splits = 1; splits <= 2 && splits <= batches; ++splits) {
+      const double there = cost(tall, splits, 7.4, 37.5);
+      if (there < best) {
+        best = there;
+        p = {0, fx::kTallRowTiles, 0, splits, 0, true};
+      }
+    }
+  }
   p.batches_per_split = (batches + p.splits - 1) / p.splits;
   p.splits = (batches + p.batches_per_split - 1) / p.batches_per_split;
   return p;
@@ -1236,9 +1230,7 @@ int fx_w3_gemm(const void* x, int x_dtype, const uint8_t* planes, const void* sc
   const fx::GemmPlan plan = gemm_plan(M, O, G);
   const size_t packed = gemm_packed_bytes(M, G, plan);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int rows = 4;  // staged rows of the permuted packing: at most 64 KB of LDS
-  while (rows > 1 && size_t(rows) * K * 2 > 65536) rows >>= 1;
-  fx::launch_gemm_pack({static_cast<const uint16_t*>(x), perm, static_cast<uint4*>(workspace), M, K, plan.mt, rows}, s);
+  fx::launch_gemm_pack({static_cast<const uint16_t*>(x), perm, static_cast<uint4*>(workspace), M, K, plan.mt}, s);
   rc = check_launch("gemm_pack_kernel");
   if (rc) return rc;
   fx::GemmArgs a{};
@@ -1253,7 +1245,8 @@ int fx_w3_gemm(const void* x, int x_dtype, const uint8_t* planes, const void* sc
   a.batches_per_split = plan.batches_per_split;
   a.vec = O % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
   const bool wide = plan.mt >= 4, bf = x_dtype == FX_BF16;
-  const bool ran = wide ? (bf ? fx::dispatch_gemm_wide_bf16(plan, a, s) : fx::dispatch_gemm_wide_f16(plan, a, s))
+  const bool ran = plan.tall ? (bf ? fx::dispatch_gemm_tall_bf16(plan, a, s) : fx::dispatch_gemm_tall_f16(plan, a, s))
+                 : wide ? (bf ? fx::dispatch_gemm_wide_bf16(plan, a, s) : fx::dispatch_gemm_wide_f16(plan, a, s))
                         : (bf ? fx::dispatch_gemm_bf16(plan, a, s) : fx::dispatch_gemm_f16(plan, a, s));
   if (!ran) return fail(FX_EINVAL, "no GEMM kernel for plan (%d, %d, %d)", plan.rt, plan.mt, plan.nk);
   rc = check_launch("w3_gemm_kernel");

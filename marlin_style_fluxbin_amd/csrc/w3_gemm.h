@@ -30,59 +30,9 @@
 #pragma once
 #include "w3_gemm_launch.h"
 #include "w3_mfma.hip"
+#include "w3_values.h"
 
 namespace fx {
-
-// The eight values of one (row, group), as bytes for v_perm_b32: l0 / l1 the low
-// bytes of codes 0..3 / 4..7, h0 / h1 the high bytes.
-struct ValueTable {
-  unsigned l0, l1, h0, h1;
-};
-
-template <int XDT>
-__device__ __forceinline__ ValueTable value_table(unsigned scale_bits, unsigned zero, int sdt) {
-  const float s = sdt == kBF16 ? to_f32<kBF16>(uint16_t(scale_bits)) : to_f32<kF16>(uint16_t(scale_bits));
-  const float z = float(zero);
-  unsigned p[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float a = s * (float(2 * i) - z), b = s * (float(2 * i + 1) - z);
-    if (sdt != XDT) {  // round to the scale's type first, as the restored weight does
-      if (sdt == kBF16) round_pair<kBF16>(a, b);
-      else round_pair<kF16>(a, b);
-    }
-    p[i] = round_pair_bits<XDT>(a, b);
-  }
-  return ValueTable{__builtin_amdgcn_perm(p[1], p[0], 0x06040200u), __builtin_amdgcn_perm(p[3], p[2], 0x06040200u),
-                    __builtin_amdgcn_perm(p[1], p[0], 0x07050301u), __builtin_amdgcn_perm(p[3], p[2], 0x07050301u)};
-}
-
-// T_s of dequant_word: the code of column 4 n + s in bits 4 n .. 4 n + 2.
-__device__ __forceinline__ void code_words(unsigned p0, unsigned p1, unsigned p2, unsigned (&t)[4]) {
-  const unsigned M0 = 0x11111111u, M1 = 0x22222222u;
-  t[0] = select3(p0, p1 << 1, p2 << 2, M0, M1);
-  t[1] = select3(p0 >> 1, p1, p2 << 1, M0, M1);
-  t[2] = select3(p0 >> 2, p1 >> 1, p2, M0, M1);
-  t[3] = select3(p0 >> 3, p1 >> 2, p2 >> 1, M0, M1);
-}
-
-// A operands of steps b = ODD and b = ODD + 2 of one word: element e of step b is
-// column 8 b + e.
-template <bool ODD>
-__device__ __forceinline__ void expand_steps(const unsigned (&t)[4], const ValueTable& v, u32x4_t& a0, u32x4_t& a2) {
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {  // columns 2 i, 2 i + 1 (low nibbles) and 4 + 2 i, 5 + 2 i (high)
-    const unsigned both = ODD ? __builtin_amdgcn_bitop3_b32(t[2 * i] >> 8, t[2 * i + 1], 0x00ff00ffu, 0xE4)
-                              : __builtin_amdgcn_bitop3_b32(t[2 * i], t[2 * i + 1] << 8, 0x00ff00ffu, 0xE4);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const unsigned sel = (h ? both >> 4 : both) & 0x07070707u;
-      const unsigned lo = __builtin_amdgcn_perm(v.l1, v.l0, sel), hi = __builtin_amdgcn_perm(v.h1, v.h0, sel);
-      a0[2 * h + i] = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
-      a2[2 * h + i] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
-    }
-  }
-}
 
 template <int XDT>
 __device__ __forceinline__ f32x4_t mfma16(const u32x4_t& a, const u32x4_t& b, const f32x4_t& d) {
@@ -92,6 +42,53 @@ __device__ __forceinline__ f32x4_t mfma16(const u32x4_t& a, const u32x4_t& b, co
   else
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), d, 0,
                                                   0, 0);
+}
+
+// A wave's outputs (or its split's partials).
+template <int XDT, int RT, int MT>
+__device__ __forceinline__ void gemm_store(const GemmArgs& a, const f32x4_t (&acc)[RT][MT], int row0, int m0, int r,
+                                           int kb) {
+  // lane (r, kb): rows 4 kb .. + 3 of each tile, activation row m0 + 16 mt + r
+#pragma unroll
+  for (int tt = 0; tt < RT; ++tt) {
+    const int o = row0 + 16 * tt + 4 * kb;
+    if (o >= a.O) continue;
+    float bias[4] = {0.f, 0.f, 0.f, 0.f};
+    if (a.bias && !a.partial) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (o + j < a.O) bias[j] = to_f32<XDT>(a.bias[o + j]);
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int m = m0 + 16 * mt + r;
+      if (m >= a.M) continue;
+      const f32x4_t d = acc[tt][mt];
+      if (a.partial) {
+        float* dst = a.partial + (size_t(blockIdx.z) * a.M + m) * a.O + o;
+        if (a.vec) {
+          *reinterpret_cast<f32x4_t*>(dst) = d;
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (o + j < a.O) dst[j] = d[j];
+        }
+      } else {
+        uint16_t* dst = a.out + size_t(m) * a.O + o;
+        uint16_t v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = from_f32<XDT>(d[j] + bias[j]);
+        if (a.vec) {
+          *reinterpret_cast<uint2*>(dst) =
+              uint2{unsigned(v[0]) | (unsigned(v[1]) << 16), unsigned(v[2]) | (unsigned(v[3]) << 16)};
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (o + j < a.O) dst[j] = v[j];
+        }
+      }
+    }
+  }
 }
 
 template <int XDT, int RT, int MT, int NK, int PD, bool NEXT>
@@ -223,47 +220,7 @@ __global__ __launch_bounds__(NK * 64) void w3_gemm_kernel(GemmArgs a) {
     __syncthreads();
   }
   if (part > 0) return;
-  // lane (r, kb): rows 4 kb .. + 3 of each tile, activation row m0 + 16 mt + r
-#pragma unroll
-  for (int tt = 0; tt < RT; ++tt) {
-    const int o = row0 + 16 * tt + 4 * kb;
-    if (o >= a.O) continue;
-    float bias[4] = {0.f, 0.f, 0.f, 0.f};
-    if (a.bias && !a.partial) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (o + j < a.O) bias[j] = to_f32<XDT>(a.bias[o + j]);
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = m0 + 16 * mt + r;
-      if (m >= a.M) continue;
-      const f32x4_t d = acc[tt][mt];
-      if (a.partial) {
-        float* dst = a.partial + (size_t(blockIdx.z) * a.M + m) * a.O + o;
-        if (a.vec) {
-          *reinterpret_cast<f32x4_t*>(dst) = d;
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (o + j < a.O) dst[j] = d[j];
-        }
-      } else {
-        uint16_t* dst = a.out + size_t(m) * a.O + o;
-        uint16_t v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = from_f32<XDT>(d[j] + bias[j]);
-        if (a.vec) {
-          *reinterpret_cast<uint2*>(dst) =
-              uint2{unsigned(v[0]) | (unsigned(v[1]) << 16), unsigned(v[2]) | (unsigned(v[3]) << 16)};
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (o + j < a.O) dst[j] = v[j];
-        }
-      }
-    }
-  }
+  gemm_store<XDT, RT, MT>(a, acc, row0, m0, r, kb);
 }
 
 template <int XDT, int RT, int MT, int NK, int PD, bool NEXT>

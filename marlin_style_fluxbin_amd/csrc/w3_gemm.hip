@@ -29,52 +29,65 @@ __global__ __launch_bounds__(256) void gemm_pack_kernel(GemmPackArgs a) {
   for (int i = 0; i < 4; ++i) a.packed[packed_unit(row, c0 + i, a.mt, batches)] = v[i];
 }
 
-// With a column permutation: a workgroup copies `rows` rows into LDS and gathers the
-// units of its share of the columns from there (random 2-byte reads of HBM would
-// cost a cache line each).  Entries outside [0, K) read zero.
+// With a column permutation: a workgroup copies R rows into LDS and gathers its share
+// of the columns from there (random 2-byte reads of HBM would cost a cache line each).
+// Entries outside [0, K) read zero.
 constexpr int kPackThreads = 512;
+template <int R>
 __global__ __launch_bounds__(kPackThreads) void gemm_pack_permuted_kernel(GemmPackArgs a) {
   extern __shared__ uint4 pack_rows[];
-  const int batches = (a.K + 511) / 512, row0 = int(blockIdx.x) * a.rows, vecs = a.K / 8;
-  for (int i = threadIdx.x; i < a.rows * vecs; i += kPackThreads) {
-    const int row = row0 + i / vecs;
-    pack_rows[i] = row < a.M ? reinterpret_cast<const uint4*>(a.x)[size_t(row) * vecs + i % vecs] : make_uint4(0, 0, 0, 0);
-  }
+  const int batches = (a.K + 511) / 512, row0 = int(blockIdx.x) * R, vecs = a.K / 8;
+  const int cols = batches * 64, per = (cols + int(gridDim.y) - 1) / int(gridDim.y);  // 8-column units, units a share
+  const int c0 = int(blockIdx.y) * per, c1 = min(cols, c0 + per);
+  const int rr = int(threadIdx.x) % R, cstep = kPackThreads / R;
+  int c = c0 + int(threadIdx.x) / R;  // neighbouring lanes: rows of one unit, contiguous in the output
+  const uint4 zero = make_uint4(0, 0, 0, 0);
+  const uint4* perm = reinterpret_cast<const uint4*>(a.perm);
+  uint4 p = c < c1 && c < vecs ? perm[c] : zero;  // in flight over the copy
+  const uint4* src = reinterpret_cast<const uint4*>(a.x) + size_t(row0) * vecs;
+#pragma unroll
+  for (int k = 0; k < R; ++k)
+    for (int i = threadIdx.x; i < vecs; i += kPackThreads) pack_rows[k * vecs + i] = row0 + k < a.M ? src[k * vecs + i] : zero;
   __syncthreads();
-  const uint16_t* staged = reinterpret_cast<const uint16_t*>(pack_rows);
-  const int units = batches * 64 * a.rows;
-  const int per = (units + int(gridDim.y) - 1) / int(gridDim.y);
-  const int end = min(units, (int(blockIdx.y) + 1) * per);
-  for (int u = int(blockIdx.y) * per + int(threadIdx.x); u < end; u += kPackThreads) {
-    const int rr = u % a.rows, c = u / a.rows;  // neighbouring lanes: rows of one unit, contiguous in the output
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (c * 8 < a.K) {
-      const uint4 p = reinterpret_cast<const uint4*>(a.perm)[c];
+  const uint16_t* row = reinterpret_cast<const uint16_t*>(pack_rows + rr * vecs);
+  uint4* dst = a.packed + packed_unit(row0, 0, a.mt, batches) + rr;
+  while (c < c1) {
+    const int next = c + cstep;
+    const uint4 pn = next < c1 && next < vecs ? perm[next] : zero;
+    uint4 v = zero;
+    if (c < vecs) {
       const unsigned pw[4] = {p.x, p.y, p.z, p.w};
       unsigned o[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int lo = int(int16_t(pw[i])), hi = int(pw[i]) >> 16;
-        const unsigned a0 = unsigned(lo) < unsigned(a.K) ? staged[rr * a.K + lo] : 0u;
-        const unsigned a1 = unsigned(hi) < unsigned(a.K) ? staged[rr * a.K + hi] : 0u;
+        const unsigned a0 = unsigned(lo) < unsigned(a.K) ? row[lo] : 0u;
+        const unsigned a1 = unsigned(hi) < unsigned(a.K) ? row[hi] : 0u;
         o[i] = a0 | (a1 << 16);
       }
       v = make_uint4(o[0], o[1], o[2], o[3]);
     }
-    a.packed[packed_unit(row0 + rr, c, a.mt, batches)] = v;
+    dst[size_t(((c >> 6) * 16 + (c & 15)) * a.mt) * 64 + ((c >> 4) & 3) * 16] = v;
+    c = next;
+    p = pn;
   }
 }
 
+// Rows a workgroup stages: four write 64 contiguous bytes of the output together;
+// few rows run one to a workgroup, shared over more of them, since their copy and
+// gather are then the latency (37 rows of 4096: 4.8 us with four, see the kernel trace).
 void launch_gemm_pack(const GemmPackArgs& a, hipStream_t s) {
-  const int batches = (a.K + 511) / 512, tiles = (a.M + 16 * a.mt - 1) / (16 * a.mt) * a.mt;
+  const int batches = (a.K + 511) / 512, tiles = (a.M + 16 * a.mt - 1) / (16 * a.mt) * a.mt, rows = tiles * 16;
   if (!a.perm) {
     hipLaunchKernelGGL(gemm_pack_kernel, dim3(unsigned(tiles * batches)), dim3(256), 0, s, a);
     return;
   }
-  const int blocks = tiles * 16 / a.rows;
-  const int share = blocks < 64 ? 4 : blocks < 256 ? 2 : 1;  // workgroups that share the columns of the same rows
-  hipLaunchKernelGGL(gemm_pack_permuted_kernel, dim3(unsigned(blocks), unsigned(share)), dim3(kPackThreads),
-                     size_t(a.rows) * a.K * 2, s, a);
+  const int want = rows <= 64 ? 1 : rows <= 128 ? 2 : 4, fits = 65536 / (2 * a.K);  // at most 64 KB of LDS
+  const int r = want == 4 && fits >= 4 ? 4 : want >= 2 && fits >= 2 ? 2 : 1;
+  const unsigned blocks = unsigned(rows / r), share = blocks < 128 ? 4 : blocks < 256 ? 2 : 1;
+  const auto kernel = r == 4 ? gemm_pack_permuted_kernel<4> : r == 2 ? gemm_pack_permuted_kernel<2>
+                                                                   : gemm_pack_permuted_kernel<1>;
+  hipLaunchKernelGGL(kernel, dim3(blocks, share), dim3(kPackThreads), size_t(r) * a.K * 2, s, a);
 }
 
 // out = the splits' partials in split order, plus the bias, rounded once; four

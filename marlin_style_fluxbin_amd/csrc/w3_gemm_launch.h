@@ -27,7 +27,6 @@ struct GemmPackArgs {
   const int16_t* perm;  // [K] (16-byte aligned) or null: the identity
   uint4* packed;
   int M, K, mt;         // mt: 16-row tiles per row block
-  int rows;             // perm: rows a workgroup stages (a divisor of 16)
 };
 
 // A tiling: rt 16-row output tiles x mt 16-row activation tiles per workgroup, nk
@@ -35,7 +34,9 @@ struct GemmPackArgs {
 struct GemmPlan {
   int rt, mt, nk;
   int splits, batches_per_split;
+  bool tall;  // w3_gemm_tall.h: kTallTiles kTallWaves output tiles x kTallRowTiles
 };
+constexpr int kTallTiles = 3, kTallWaves = 4, kTallRowTiles = 8;
 
 // Instantiated (rt, mt, nk): (1..3, 1..3, 8) (2..3, 4, 8) (2, 7, 8) (4, 7, 4) (2, 8, 4)
 // (4, 8, 4).  False otherwise.
@@ -43,6 +44,8 @@ bool dispatch_gemm_bf16(const GemmPlan& p, const GemmArgs& a, hipStream_t s);
 bool dispatch_gemm_f16(const GemmPlan& p, const GemmArgs& a, hipStream_t s);
 bool dispatch_gemm_wide_bf16(const GemmPlan& p, const GemmArgs& a, hipStream_t s);
 bool dispatch_gemm_wide_f16(const GemmPlan& p, const GemmArgs& a, hipStream_t s);
+bool dispatch_gemm_tall_bf16(const GemmPlan& p, const GemmArgs& a, hipStream_t s);
+bool dispatch_gemm_tall_f16(const GemmPlan& p, const GemmArgs& a, hipStream_t s);
 void launch_gemm_pack(const GemmPackArgs& a, hipStream_t s);
 void launch_gemm_finish(int xdt, const GemmArgs& a, int splits, hipStream_t s);
 

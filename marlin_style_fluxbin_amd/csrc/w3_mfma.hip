@@ -47,6 +47,7 @@
 #pragma once
 #include "common.h"
 #include "w3_mfma_launch.h"
+#include "w3_values.h"
 
 namespace fx {
 
@@ -86,16 +87,6 @@ __device__ __forceinline__ uint16_t exact_bits(float v) {
 // from P1 and the remaining bits from the un-inverted plane 2.
 __device__ __forceinline__ unsigned bitfield_insert(unsigned mask, unsigned a, unsigned b) {
   return (a & mask) | (b & ~mask);  // v_bfi_b32
-}
-
-// T_s from three-input bit operations (v_bitop3_b32, gfx950): u = M1 ? b : ~c
-// (table 0xB1, operand order b, c, m: the inversion of stored plane 2 folded in),
-// then T = M0 ? a : u (table 0xE4).  The complement of the shifted plane differs
-// from the shifted complement only in shifted-in bits, which land in bits the
-// masks take from the other planes or in the don't-care bit.  Two instructions
-// per T_s where the compiler's own rewrite of the inserts took three to four.
-__device__ __forceinline__ unsigned select3(unsigned a, unsigned b, unsigned c, unsigned m0, unsigned m1) {
-  return __builtin_amdgcn_bitop3_b32(a, __builtin_amdgcn_bitop3_b32(b, c, m1, 0xB1), m0, 0xE4);
 }
 
 __device__ __forceinline__ void dequant_word(unsigned p0, unsigned p1, unsigned p2, u32x4_t a[4]) {

@@ -57,7 +57,8 @@ def test_gemm_tiles(gpu, m, o, k, dtype, scale):
 
 
 @pytest.mark.parametrize("m,o,k", [(12, 9216, 512), (20, 9217, 256), (40, 12288, 640), (60, 9230, 512),
-                                   (112, 12288, 256), (128, 12300, 512), (400, 4096, 1024), (1024, 1500, 512),
+                                   (112, 12288, 256), (128, 12300, 512), (400, 4096, 1024), (512, 1500, 512),
+                                   (510, 12288, 640), (300, 12210, 1408), (400, 9000, 128), (500, 4100, 8192),
                                    (37, 512, 12288), (64, 1024, 12288), (100, 300, 16384), (200, 700, 8192)])
 def test_gemm_wide_and_split_plans(gpu, m, o, k):
     module = _module(gpu, o, k, seed=3, permute=True)
