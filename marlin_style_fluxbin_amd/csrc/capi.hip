@@ -18,6 +18,7 @@
 #include "two_base_launch.h"
 #include "w3_gemm_launch.h"
 #include "w3_restore_launch.h"
+#include "w3_split_launch.h"
 
 using fx::LutArgs;
 using fx::MfmaArgs;
@@ -147,6 +148,32 @@ int run_lut(const void* x, int x_dtype, const uint8_t* planes, const void* scale
     done += mb;
   }
   return FX_OK;
+}
+
+// One row on the matrix cores where the kernel forms these splits (w3_split.hip), else
+// the table kernel.  out null: partials only; partial null: one split.
+bool run_split(const void* x, int x_dtype, const uint8_t* planes, const void* scales, int scale_dtype,
+               const uint8_t* zeros, const int16_t* perm, float* partial, void* out, int M, int O, int K, int gps,
+               int arithmetic, hipStream_t stream, int* rc) {
+  const int G = K / 128;
+  if (M != 1 || !fx::split_kernel_takes(G, gps)) return false;
+  const fx::SplitArgs a{static_cast<const uint16_t*>(x),
+                        planes,
+                        static_cast<const uint16_t*>(scales),
+                        zeros,
+                        perm,
+                        partial,
+                        static_cast<uint16_t*>(out),
+                        O,
+                        G,
+                        gps,
+                        scale_dtype,
+                        arithmetic == FX_ARITH_DECODED_BF16,
+                        reinterpret_cast<uintptr_t>(x) % 16 == 0,
+                        reinterpret_cast<uintptr_t>(perm) % 16 == 0};
+  fx::launch_split(x_dtype, a, stream);
+  *rc = check_launch("w3_split_kernel");
+  return true;
 }
 
 int launch_finish(const float* partial, void* out, int out_dtype, int splits, int MO,
@@ -587,6 +614,9 @@ int fx_w3_inline_main(const void* x, int x_dtype, const uint8_t* planes, const v
   if (groups_per_split < 1 || groups_per_split > G)
     return fail(FX_EINVAL, "groups_per_split must be in [1, K/128]");
   if (lut_block_for(M) != M) return fail(FX_EINVAL, "inline_main supports M in {1,2,4,8}");
+  if (run_split(x, x_dtype, planes, scales, scale_dtype, zeros, perm, partial, nullptr, M, O, K, groups_per_split,
+                arithmetic, static_cast<hipStream_t>(stream), &rc))
+    return rc;
   return run_lut(x, x_dtype, planes, scales, scale_dtype, zeros, perm, partial, nullptr, M, O, K,
                  arithmetic, make_lut_tile(O, G, rpt, groups_per_split), true,
                  static_cast<hipStream_t>(stream));
@@ -615,10 +645,13 @@ int fx_w3_m1_out(const void* x, int x_dtype, const uint8_t* planes, const void* 
   if (lut_block_for(M) != M) return fail(FX_EINVAL, "m1_out supports M in {1,2,4,8}");
   const LutTile tile = make_lut_tile(O, G, rpt, groups_per_split);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (tile.splits > 1 && !workspace) return fail(FX_EINVAL, "workspace must be non-null when K is split");
+  if (run_split(x, x_dtype, planes, scales, scale_dtype, zeros, perm, tile.splits > 1 ? workspace : nullptr, out, M, O, K,
+                groups_per_split, arithmetic, s, &rc))
+    return rc;
   if (tile.splits == 1)
-    return run_lut(x, x_dtype, planes, scales, scale_dtype, zeros, perm, nullptr, out, M, O, K,
-                   arithmetic, tile, false, s);
-  if (!workspace) return fail(FX_EINVAL, "workspace must be non-null when K is split");
+    return run_lut(x, x_dtype, planes, scales, scale_dtype, zeros, perm, nullptr, out, M, O, K, arithmetic, tile, false,
+                   s);
   rc = run_lut(x, x_dtype, planes, scales, scale_dtype, zeros, perm, workspace, nullptr, M, O, K,
                arithmetic, tile, true, s);
   if (rc) return rc;

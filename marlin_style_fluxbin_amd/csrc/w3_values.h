@@ -25,6 +25,12 @@ struct ValueTable {
   unsigned l0, l1, h0, h1;
 };
 
+// The table of eight 16-bit values, two per word.
+__device__ __forceinline__ ValueTable table_of_pairs(const unsigned (&p)[4]) {
+  return ValueTable{__builtin_amdgcn_perm(p[1], p[0], 0x06040200u), __builtin_amdgcn_perm(p[3], p[2], 0x06040200u),
+                    __builtin_amdgcn_perm(p[1], p[0], 0x07050301u), __builtin_amdgcn_perm(p[3], p[2], 0x07050301u)};
+}
+
 template <int XDT>
 __device__ __forceinline__ ValueTable value_table(unsigned scale_bits, unsigned zero, int sdt) {
   const float s = sdt == kBF16 ? to_f32<kBF16>(uint16_t(scale_bits)) : to_f32<kF16>(uint16_t(scale_bits));
@@ -39,8 +45,7 @@ __device__ __forceinline__ ValueTable value_table(unsigned scale_bits, unsigned 
     }
     p[i] = round_pair_bits<XDT>(a, b);
   }
-  return ValueTable{__builtin_amdgcn_perm(p[1], p[0], 0x06040200u), __builtin_amdgcn_perm(p[3], p[2], 0x06040200u),
-                    __builtin_amdgcn_perm(p[1], p[0], 0x07050301u), __builtin_amdgcn_perm(p[3], p[2], 0x07050301u)};
+  return table_of_pairs(p);
 }
 
 // T_s of dequant_word: the code of column 4 n + s in bits 4 n .. 4 n + 2.
