@@ -127,7 +127,10 @@ def ptr(tensor: torch.Tensor | None) -> int | None:
 
 
 def stream_handle(device: torch.device | None = None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream of ``device`` (default: the current device) as an integer,
+    without building a ``torch.cuda.Stream`` for it (2.6 us of every call)."""
+    index = None if device is None else device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def require_gpu_tensor(tensor: torch.Tensor, name: str) -> None:

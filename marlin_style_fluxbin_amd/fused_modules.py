@@ -45,7 +45,13 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
 
 def _hip_ok(*tensors: torch.Tensor) -> bool:
     first = tensors[0]
-    return first.is_cuda and first.dtype in _HALF and all(t.dtype == first.dtype for t in tensors)
+    dtype = first.dtype
+    if not first.is_cuda or dtype not in _HALF:
+        return False
+    for t in tensors:
+        if t.dtype != dtype:
+            return False
+    return True
 
 
 def rms_norm(hidden_states: torch.Tensor, weight: torch.Tensor, eps: float, *,
@@ -59,10 +65,11 @@ def rms_norm(hidden_states: torch.Tensor, weight: torch.Tensor, eps: float, *,
     x = _aligned(hidden_states)
     w = _aligned(weight)
     result = out if out is not None else torch.empty_like(x)
-    lib = _lib.library()
-    _lib.check(lib.fx_rmsnorm(x.data_ptr(), None, w.data_ptr(), result.data_ptr(), None,
-                              x.numel() // hidden, hidden, float(eps), _lib.dtype_code(x.dtype),
-                              _lib.stream_handle(x.device)), "fx_rmsnorm")
+    rc = _lib.library().fx_rmsnorm(x.data_ptr(), None, w.data_ptr(), result.data_ptr(), None,
+                                   x.numel() // hidden, hidden, float(eps), _lib.dtype_code(x.dtype),
+                                   _lib.stream_handle(x.device))
+    if rc:
+        _lib.check(rc, "fx_rmsnorm")
     return result
 
 

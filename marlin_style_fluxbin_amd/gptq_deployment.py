@@ -171,25 +171,27 @@ def validate_planar_w3(layout: Mapping[str, torch.Tensor], *, check_values: bool
     devices and contiguity only.  The full form adds finite scales, zero-points
     in [0, 7] and a bijective ``perm``.
     """
-    keys = set(layout)
-    if keys != set(FIELDS) and keys != set(FIELDS) | set(OPTIONAL_FIELDS):
+    zeros = layout.get("zeros")
+    if len(layout) != len(FIELDS) + (zeros is not None) or any(name not in layout for name in FIELDS):
         raise ValueError(f"expected exactly {FIELDS} (+ optional {OPTIONAL_FIELDS})")
     planes, scales, perm = (layout[name] for name in FIELDS)
-    if planes.dtype != torch.uint8 or planes.ndim != 4 or planes.shape[1] != 3 or planes.shape[3] != 16:
+    shape = planes.shape
+    if planes.dtype != torch.uint8 or len(shape) != 4 or shape[1] != 3 or shape[3] != 16:
         raise ValueError("planes must be uint8 [G,3,O,16]")
-    groups, _, out_features, _ = planes.shape
-    if scales.dtype not in SCALE_DTYPES or tuple(scales.shape) != (groups, out_features):
+    groups, _, out_features, _ = shape
+    if scales.dtype not in SCALE_DTYPES or scales.shape != (groups, out_features):
         raise ValueError("deployment scales must be bfloat16 or float16 [G,O]")
     in_features = groups * GROUP_SIZE
     if in_features > 32767:
         raise ValueError("perm indices must be representable by int16")
-    if perm.dtype != torch.int16 or tuple(perm.shape) != (in_features,):
+    if perm.dtype != torch.int16 or perm.shape != (in_features,):
         raise ValueError("perm must be int16 [K]")
-    zeros = layout.get("zeros")
-    if zeros is not None and (zeros.dtype != torch.uint8 or tuple(zeros.shape) != (groups, out_features)):
+    if zeros is not None and (zeros.dtype != torch.uint8 or zeros.shape != (groups, out_features)):
         raise ValueError("zeros must be uint8 [G,O]")
-    if any(value.device != planes.device or not value.is_contiguous() for value in layout.values()):
-        raise ValueError("layout tensors must be contiguous on one device")
+    device = planes.device
+    for value in layout.values():
+        if value.device != device or not value.is_contiguous():
+            raise ValueError("layout tensors must be contiguous on one device")
     if check_values:
         if not torch.isfinite(scales).all():
             raise ValueError("scales must be finite")

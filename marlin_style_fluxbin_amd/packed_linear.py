@@ -104,8 +104,9 @@ class PackedLinearBase(nn.Module):
         """Drop cached kernel bindings that hold device pointers."""
 
     def _count(self, route: str) -> None:
-        self.route_counts[route] = self.route_counts.get(route, 0) + 1
-        self.last_route = route
+        counts = self.route_counts
+        counts[route] = counts.get(route, 0) + 1
+        object.__setattr__(self, "last_route", route)  # a str: no module bookkeeping to do
 
     def reset_route_counts(self) -> None:
         """Zero every route counter this module keeps (``packed_small_m`` too,
@@ -148,16 +149,15 @@ class PackedLinearBase(nn.Module):
     def _packed_rows(self, x: torch.Tensor) -> int:
         """Row count if ``x`` may take the packed route, else 0."""
         rows = x.numel() // self.in_features
-        if x.is_cuda and x.dtype in HALF_DTYPES and 1 <= rows <= self.max_packed_rows:
-            return rows
-        return 0
+        return rows if 1 <= rows <= self.max_packed_rows and x.is_cuda and x.dtype in HALF_DTYPES else 0
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self._decode_binding is not None:
             return self._decode_binding(x)
         if torch.is_grad_enabled():
             raise RuntimeError("packed inference requires no_grad/inference_mode")
-        if x.ndim < 2 or x.shape[-1] != self.in_features:
+        shape, k = x.shape, self.in_features
+        if len(shape) < 2 or shape[-1] != k:
             raise ValueError("expected [...,K] input")
         self._check_before_call()
         rows = self._packed_rows(x)
@@ -167,11 +167,14 @@ class PackedLinearBase(nn.Module):
             self._count(DENSE_FALLBACK)
             return self._dense_linear(x)
         self._count(PACKED_M1 if rows == 1 else PACKED_SMALL_M)
-        out = torch.empty((rows, self.out_features), device=x.device, dtype=x.dtype)
-        self._packed_kernel(rows, x.device)(x.reshape(rows, self.in_features).contiguous(), out)
-        if self.bias is not None:
-            out = out.add_(self.bias) if self.bias_in_place else out + self.bias
-        return out.reshape(*x.shape[:-1], self.out_features)
+        device, o = x.device, self.out_features
+        flat = len(shape) == 2
+        out = torch.empty((rows, o), device=device, dtype=x.dtype)
+        self._packed_kernel(rows, device)((x if flat else x.reshape(rows, k)).contiguous(), out)
+        bias = self._buffers["bias"]
+        if bias is not None:
+            out = out.add_(bias) if self.bias_in_place else out + bias
+        return out if flat else out.reshape(*shape[:-1], o)
 
 
 def replace_linears_atomically(block: nn.Module, built: list[tuple[str, nn.Module]]) -> list[str]:

@@ -368,12 +368,13 @@ class W3Gemv:
         self.workspace = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=device)
 
     def __call__(self, x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
-        m = x.shape[0]
-        _lib.check(self.lib.fx_w3_gemv(
-            x.data_ptr(), _lib.dtype_code(x.dtype), self.layout["planes"].data_ptr(),
-            self.layout["scales"].data_ptr(), self.scale_code, self.zeros_ptr, self.perm_ptr,
-            self.workspace.data_ptr(), self.workspace.numel(), out.data_ptr(), m, self.out_features,
-            self.in_features, self.arith, _lib.stream_handle(x.device)), "fx_w3_gemv")
+        layout, workspace = self.layout, self.workspace
+        rc = self.lib.fx_w3_gemv(
+            x.data_ptr(), _lib.dtype_code(x.dtype), layout["planes"].data_ptr(), layout["scales"].data_ptr(),
+            self.scale_code, self.zeros_ptr, self.perm_ptr, workspace.data_ptr(), workspace.numel(), out.data_ptr(),
+            x.shape[0], self.out_features, self.in_features, self.arith, _lib.stream_handle(x.device))
+        if rc:
+            _lib.check(rc, "fx_w3_gemv")
         return out
 
 
@@ -452,7 +453,8 @@ class PackedW3Linear(PackedLinearBase):
         return self.groups_per_split != 1
 
     def layout(self) -> dict:
-        return {name: getattr(self, name) for name in self._fields}
+        buffers = self._buffers
+        return {name: buffers[name] for name in self._fields}
 
     def _payload_device(self) -> torch.device:
         return self.planes.device
@@ -463,32 +465,41 @@ class PackedW3Linear(PackedLinearBase):
     def _gemm_takes(self, x: torch.Tensor) -> bool:
         """The dense-fallback inputs that ``fx_w3_gemm`` multiplies; the restored
         weight and ``F.linear`` take (or refuse) every other one."""
-        planes, bias = self.planes, self.bias
+        buffers = self._buffers
+        planes, bias = buffers["planes"], buffers["bias"]
         return (x.is_cuda and x.dtype in HALF_DTYPES and x.device == planes.device and plain_call(x)
                 and 0 < x.numel() <= GEMM_MAX_ROWS * self.in_features
-                and planes.numel() < 2**31 and planes.data_ptr() % 16 == 0 and self.perm.data_ptr() % 16 == 0
+                and planes.numel() < 2**31 and planes.data_ptr() % 16 == 0 and buffers["perm"].data_ptr() % 16 == 0
                 and (bias is None or (bias.dtype == x.dtype and bias.device == x.device and bias.is_contiguous())))
 
     def _dense_linear(self, x: torch.Tensor) -> torch.Tensor:
         if self._gemm_takes(x):
-            rows = x.numel() // self.in_features
-            flat = x.reshape(rows, self.in_features).contiguous()
+            shape, k = x.shape, self.in_features
+            if len(shape) == 2:
+                flat, rows = x.contiguous(), shape[0]
+            else:
+                rows = x.numel() // k
+                flat = x.reshape(rows, k).contiguous()
             if flat.data_ptr() % 16 == 0:
-                return self._gemm(flat, rows).view(*x.shape[:-1], self.out_features)
+                y = self._gemm(flat, rows)
+                return y if len(shape) == 2 else y.view(*shape[:-1], self.out_features)
         return super()._dense_linear(x)
 
     def _gemm(self, x: torch.Tensor, rows: int) -> torch.Tensor:
         layout = self.layout()
-        validate_planar_w3(layout, check_values=False)
-        lib, o, k = _lib.library(), self.out_features, self.in_features
-        out = torch.empty((rows, o), dtype=x.dtype, device=x.device)
+        o, k = validate_planar_w3(layout, check_values=False)
+        lib, device, dtype = _lib.library(), x.device, x.dtype
+        out = torch.empty((rows, o), dtype=dtype, device=device)
         nbytes = lib.fx_w3_gemm_workspace_bytes(rows, o, k)
-        workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-        _lib.check(lib.fx_w3_gemm(
-            x.data_ptr(), _lib.dtype_code(x.dtype), self.planes.data_ptr(), self.scales.data_ptr(),
-            _lib.dtype_code(self.scales.dtype), _lib.ptr(layout.get("zeros")),
-            None if self._perm_identity else self.perm.data_ptr(), _lib.ptr(self.bias), workspace.data_ptr(), nbytes,
-            out.data_ptr(), rows, o, k, _lib.stream_handle(x.device)), "fx_w3_gemm")
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        scales = layout["scales"]
+        rc = lib.fx_w3_gemm(
+            x.data_ptr(), _lib.dtype_code(dtype), layout["planes"].data_ptr(), scales.data_ptr(),
+            _lib.dtype_code(scales.dtype), _lib.ptr(layout.get("zeros")),
+            None if self._perm_identity else layout["perm"].data_ptr(), _lib.ptr(self._buffers["bias"]),
+            workspace.data_ptr(), nbytes, out.data_ptr(), rows, o, k, _lib.stream_handle(device))
+        if rc:
+            _lib.check(rc, "fx_w3_gemm")
         return out
 
     def _check_before_bind(self, device: torch.device) -> None:
@@ -503,7 +514,7 @@ class PackedW3Linear(PackedLinearBase):
             if self._table is None or self._table.workspace.device != device:
                 self._table = _TableRoute(self, device)
             return self._table
-        if self._gemv is None or self._gemv.layout["planes"].data_ptr() != self.planes.data_ptr():
+        if self._gemv is None or self._gemv.layout["planes"].data_ptr() != self._buffers["planes"].data_ptr():
             self._gemv = W3Gemv(self.layout(), arithmetic=self.arithmetic, perm_identity=self._perm_identity,
                                 max_rows=self.max_packed_rows)
         return self._gemv
