@@ -154,6 +154,132 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* __restrict
   }
 }
 
+// Rows of at most 128 values (the q/k norms): 16 lanes hold a row, 8 values each.  A wave
+// per row left three quarters of its lanes without a value and one 256-byte load in
+// flight per wave: 32000 rows of 128 took 16.2 us and take 5.4 (four rows a thread: 5.8;
+// the 16 MB alone take 3.2).  The lanes past a row add zeros to its sum there, so the
+// 16-lane sum has the same bits.
+template <int DT>
+__global__ __launch_bounds__(256) void rmsnorm_narrow_kernel(const uint16_t* __restrict__ x,
+                                                             const uint16_t* __restrict__ residual,
+                                                             const uint16_t* __restrict__ weight, uint16_t* out,
+                                                             uint16_t* residual_out, int rows, int hidden, float eps) {
+  const int c = int(threadIdx.x & 15u);
+  const int row = int(blockIdx.x) * 16 + int(threadIdx.x >> 4);
+  const bool live = c * 8 < hidden && row < rows;
+  const size_t at = size_t(row) * hidden + c * 8;
+  const u32x4_t zero = {0u, 0u, 0u, 0u};
+  u32x4_t sv = live ? *reinterpret_cast<const u32x4_t*>(x + at) : zero;
+  const u32x4_t rv = live && residual ? *reinterpret_cast<const u32x4_t*>(residual + at) : zero;
+  const u32x4_t wv = live ? *reinterpret_cast<const u32x4_t*>(weight + c * 8) : zero;
+  if (residual) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float lo = rnd<DT>(to_f32<DT>(uint16_t(sv[w])) + to_f32<DT>(uint16_t(rv[w])));
+      const float hi = rnd<DT>(to_f32<DT>(uint16_t(sv[w] >> 16)) + to_f32<DT>(uint16_t(rv[w] >> 16)));
+      sv[w] = unsigned(from_f32<DT>(lo)) | (unsigned(from_f32<DT>(hi)) << 16);
+    }
+    if (live) *reinterpret_cast<u32x4_t*>(residual_out + at) = sv;
+  }
+  const float inv = rsqrtf(row16_sum(sum_sq8<DT>(sv)) / float(hidden) + eps);
+  u32x4_t yv;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const float n0 = rnd<DT>(to_f32<DT>(uint16_t(sv[w])) * inv);
+    const float n1 = rnd<DT>(to_f32<DT>(uint16_t(sv[w] >> 16)) * inv);
+    const float y0 = to_f32<DT>(uint16_t(wv[w])) * n0;
+    const float y1 = to_f32<DT>(uint16_t(wv[w] >> 16)) * n1;
+    yv[w] = unsigned(from_f32<DT>(y0)) | (unsigned(from_f32<DT>(y1)) << 16);
+  }
+  if (live) *reinterpret_cast<u32x4_t*>(out + at) = yv;
+}
+
+// RoPE (or a strided copy) of tensors without a norm, 16 bytes at a time: a thread owns
+// 8 rotate-half pairs of one position and walks kRopeHeads heads with the position's cos
+// and sin in registers.  Element by element a wave moved 256 bytes per load and divided
+// for every row: q and k of 1000 positions (40 heads of 128) took 19.4 us and take 7.7.
+// Bit for bit the torch algebra: contraction is off, since the compiler
+// otherwise forms the fp16 sum and its cast as one mixed-precision instruction with one
+// rounding.
+constexpr int kRopeHeads = 4;
+template <int DT>
+__global__ __launch_bounds__(256) void rope_vector_kernel(HeadNormRopeArgs a) {
+#pragma clang fp contract(off)
+  const int per_row = a.head_dim / 16;  // threads of a row
+  const int rows = 256 / per_row;       // positions of a workgroup
+  const int c = int(threadIdx.x) % per_row, s = int(blockIdx.x) * rows + int(threadIdx.x) / per_row;
+  int g = int(blockIdx.y), ti = 0;  // head group of tensor ti
+  while (g >= (a.t[ti].heads + kRopeHeads - 1) / kRopeHeads) {
+    g -= (a.t[ti].heads + kRopeHeads - 1) / kRopeHeads;
+    ++ti;
+  }
+  if (int(threadIdx.x) >= rows * per_row || s >= a.seq) return;
+  const HeadTensor& T = a.t[ti];
+  const int b = int(blockIdx.z), h0 = g * kRopeHeads, half = a.head_dim / 2;
+  const uint16_t* in = static_cast<const uint16_t*>(T.in) + b * T.in_stride[0] + h0 * T.in_stride[1] + s * T.in_stride[2] + 8 * c;
+  uint16_t* out = static_cast<uint16_t*>(T.out) + b * T.out_stride[0] + h0 * T.out_stride[1] + s * T.out_stride[2] + 8 * c;
+  u32x4_t lo[kRopeHeads], hi[kRopeHeads], cs[2], sn[2];
+#pragma unroll
+  for (int k = 0; k < kRopeHeads; ++k) {
+    if (h0 + k >= T.heads) break;
+    lo[k] = *reinterpret_cast<const u32x4_t*>(in + k * T.in_stride[1]);
+    hi[k] = *reinterpret_cast<const u32x4_t*>(in + k * T.in_stride[1] + half);
+  }
+  const bool rope = T.rope && a.rope_mode != kRopeNone;
+  if (rope) {
+    long long at = b * a.cs_stride[0] + s * a.cs_stride[1] + 8 * c;
+    if (a.position) at += (long long)(a.position[0]) * a.head_dim;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      cs[j] = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(a.cos) + at + j * half);
+      sn[j] = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(a.sin) + at + j * half);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kRopeHeads; ++k) {
+    if (h0 + k >= T.heads) break;
+    if (rope) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        unsigned o0 = 0, o1 = 0;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const auto at = [&](const u32x4_t& v) { return to_f32<DT>(uint16_t(v[w] >> (16 * e))); };
+          const float x0 = at(lo[k]), x1 = at(hi[k]);
+          float r0 = -x1 * at(sn[0]), r1 = x0 * at(sn[1]);  // rotate_half(y) = (-y[half:], y[:half])
+          if (a.rope_mode == kRopeStock) {
+            r0 = rnd<DT>(r0);
+            r1 = rnd<DT>(r1);
+          }
+          o0 |= unsigned(from_f32<DT>(rnd<DT>(x0 * at(cs[0])) + r0)) << (16 * e);
+          o1 |= unsigned(from_f32<DT>(rnd<DT>(x1 * at(cs[1])) + r1)) << (16 * e);
+        }
+        lo[k][w] = o0;
+        hi[k][w] = o1;
+      }
+    }
+    *reinterpret_cast<u32x4_t*>(out + k * T.out_stride[1]) = lo[k];
+    *reinterpret_cast<u32x4_t*>(out + k * T.out_stride[1] + half) = hi[k];
+  }
+}
+
+// Whether rope_vector_kernel takes a call: no norms, rows of whole 16-byte vectors whose
+// every vector is aligned.  A decode step's single position keeps the kernel below (a
+// row's 8 threads would be alone in their workgroup).
+bool rope_vector_takes(const HeadNormRopeArgs& a) {
+  if (a.seq < 8 || a.head_dim % 16 != 0 || a.head_dim > 4096) return false;
+  const auto off = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 != 0; };
+  bool rope = false;
+  for (int i = 0; i < a.ntensors; ++i) {
+    const HeadTensor& t = a.t[i];
+    if (t.weight || off(t.in) || off(t.out)) return false;
+    for (int j = 0; j < 3; ++j)
+      if (t.in_stride[j] % 8 != 0 || t.out_stride[j] % 8 != 0) return false;
+    rope = rope || (t.rope && a.rope_mode != kRopeNone);
+  }
+  return !rope || (!off(a.cos) && !off(a.sin) && a.cs_stride[0] % 8 == 0 && a.cs_stride[1] % 8 == 0);
+}
+
 // One wave per (tensor, batch, head, position) row of head_dim values.  Lane l
 // owns the rotate-half pairs (i, i + D/2) for i = l, l + 64, ... < D/2, so the
 // rotation needs no lane exchange.
@@ -228,6 +354,12 @@ __global__ __launch_bounds__(256) void head_norm_rope_kernel(HeadNormRopeArgs a)
 bool launch_rmsnorm(int dt, const uint16_t* x, const uint16_t* residual, const uint16_t* weight,
                     uint16_t* out, uint16_t* residual_out, int rows, int hidden, float eps,
                     hipStream_t s) {
+  if (dt != kBF16 && dt != kF16) return false;
+  if (hidden <= 128) {
+    hipLaunchKernelGGL(dt == kBF16 ? rmsnorm_narrow_kernel<kBF16> : rmsnorm_narrow_kernel<kF16>, dim3((rows + 15) / 16),
+                       dim3(256), 0, s, x, residual, weight, out, residual_out, rows, hidden, eps);
+    return true;
+  }
   const bool wide = hidden > 1024;
   const int rpb = wide ? 1 : 4;
   const dim3 grid((rows + rpb - 1) / rpb);
@@ -244,6 +376,18 @@ bool launch_rmsnorm(int dt, const uint16_t* x, const uint16_t* residual, const u
 }
 
 bool launch_head_norm_rope(int dt, const HeadNormRopeArgs& a, hipStream_t s) {
+  if (rope_vector_takes(a)) {
+    int groups = 0;
+    for (int i = 0; i < a.ntensors; ++i) groups += (a.t[i].heads + kRopeHeads - 1) / kRopeHeads;
+    const int positions = 256 / (a.head_dim / 16), batch = a.rows[0] / (a.t[0].heads * a.seq);
+    if (groups <= 65535 && batch <= 65535) {
+      const dim3 grid((a.seq + positions - 1) / positions, groups, batch);
+      if (dt == kBF16) hipLaunchKernelGGL(rope_vector_kernel<kBF16>, grid, dim3(256), 0, s, a);
+      else if (dt == kF16) hipLaunchKernelGGL(rope_vector_kernel<kF16>, grid, dim3(256), 0, s, a);
+      else return false;
+      return true;
+    }
+  }
   int total = 0;
   for (int i = 0; i < a.ntensors; ++i) total += a.rows[i];
   const dim3 grid((total + 3) / 4);
