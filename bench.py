@@ -204,7 +204,7 @@ def bench_shape(o, k, device, steps, warmup, stream, min_bytes=320e6, min_copies
     pout = torch.empty_like(out)
     graphs["w3_perm"] = (capture(over([lambda g=g: g(x, pout) for g in permuted]), stream), copies)
     # decoded_bf16 (the fast_corrected route: bf16 scales, zero-points 3 / 4): the
-    # MFMA kernel with the +-3 correction chain, and the reference's table kernel
+    # MFMA kernel with the +-3 correction chain, and the reference's split contract
     # (w3_lut_m1_out, one group per split) on the same payloads
     from marlin_style_fluxbin_amd.w3_lut_deployment import load_w3_lut_extension
 
@@ -322,7 +322,7 @@ def bench_shape(o, k, device, steps, warmup, stream, min_bytes=320e6, min_copies
                  zeros=decoded_views[-1]["zeros"])
     torch.cuda.synchronize()
     if not torch.allclose(dout.float(), tout.float(), rtol=2 ** -7, atol=1e-3 * float(tout.float().abs().max())):
-        raise RuntimeError("decoded_bf16 MFMA GEMV disagrees with the table kernel")
+        raise RuntimeError("decoded_bf16 MFMA GEMV disagrees with the split contract")
     batched_call(lib, xs, stacked["planes"], stacked, batch_out, o, k, _lib.PAYLOAD_PLANAR, device)
     torch.cuda.synchronize()
     if not torch.equal(batch_out[-1:], out):
@@ -959,8 +959,9 @@ def decode_bench(layers=36, prefix=512, steps=32, replays=7, seed=0):
 
 def prefill_timing(model, ids, reps=3):
     """One prefill forward of the prompt through the HF module tree (packed W3
-    Linears take their dense fallback at M > 8: the HIP restore of the weight,
-    then a hipBLASLt GEMM): HIP events around the forward, median of ``reps``
+    Linears take their dense fallback at M > 8: up to 512 rows the HIP GEMM that
+    forms the weight in registers, above them the HIP restore of the weight and a
+    hipBLASLt GEMM): HIP events around the forward, median of ``reps``
     after one untimed run."""
     import statistics
 

@@ -75,7 +75,10 @@ int fx_w3_finish(const float *partial, void *out, int out_dtype, int splits, int
 /*
  * Reference: csrc/w3_lut.cu:286-332 (m1_out), w3_lut_deployment.py:138-171.
  * With one split the workspace is not touched and one kernel writes out;
- * otherwise inline_main + finish through the fp32 workspace [splits, M, O].
+ * otherwise the partials go through the fp32 workspace [splits, M, O].  One row
+ * takes one launch on the matrix cores (groups_per_split 1, 2, a multiple of 4
+ * or all groups, K <= 16384); other calls run the table kernel, and finish
+ * where K is split.
  */
 int fx_w3_m1_out(const void *x, int x_dtype, const uint8_t *planes, const void *scales,
                  int scale_dtype, const uint8_t *zeros, const int16_t *perm, float *workspace,
@@ -90,7 +93,8 @@ int fx_w3_m1_out(const void *x, int x_dtype, const uint8_t *planes, const void *
  * accumulation, K split over the waves of a workgroup; one launch per call,
  * plus a stream-ordered finish launch when the output has fewer 16-row tiles
  * than CUs and K is also split over workgroups.  decoded_bf16 arithmetic: the
- * LUT kernel plus finish.  Tiling comes from (M, O, K) and the CU count.
+ * MFMA kernel with a correction chain for M = 1, the LUT kernel plus finish for
+ * more rows.  Tiling comes from (M, O, K) and the CU count.
  * workspace: fx_w3_gemv_workspace_bytes(M, O, K) bytes, 256-byte aligned, no
  * initial contents required; NULL is accepted when that size is 0.  Calls that
  * share a workspace must be ordered on one stream.

@@ -7,8 +7,9 @@ Both packed Linear types of the reference -- ``PackedW3Linear``
 replacers):
 
 * ``forward(x)``: a one-row fp16/bf16 GPU input takes the packed route; anything
-  else raises ``ValueError`` unless ``fallback='dense'``, which runs ``F.linear``
-  on the dequantized weight.  Both routes are counted in ``route_counts``
+  else raises ``ValueError`` unless ``fallback='dense'``, which multiplies by the
+  dequantized weight (``F.linear``, or a kernel of the subclass's that gives the same
+  product).  Both routes are counted in ``route_counts``
   (``packed_m1`` / ``dense_fallback``) and named in ``last_route``;
 * ``bind_prepared_decode(dtype)``: an allocation-free ``[1, 1, K]`` route whose
   result is a view of one module-owned output buffer, validated once at bind

@@ -11,8 +11,11 @@ Differences from the reference, all deliberate:
 * ``PackedW3Linear`` with one group per split runs the one-launch MFMA kernel in
   either arithmetic (the same sums, another fp32 order; ``decoded_bf16`` adds the
   +-3 correction as a second MFMA chain); a route that splits K over
-  ``groups_per_split > 1`` groups runs the reference's split contract on the table
-  kernel.
+  ``groups_per_split > 1`` groups runs the reference's split contract
+  (``w3_lut_m1_out``: the one-launch matrix-core kernel for the splits it forms,
+  the table kernel for the others).
+* The dense fallback of up to ``GEMM_MAX_ROWS`` rows multiplies by the restored
+  weight's values without storing them (``fx_w3_gemm``).
 * ``PackedW3Linear(max_packed_rows=n)`` opts 2..n-row inputs into the packed
   route (config 1's small-M GEMV); by default they take the dense fallback, as
   in the reference.
@@ -380,9 +383,8 @@ class W3Gemv:
 
 class _TableRoute:
     """The reference contract's packed route for one payload: ``fx_w3_m1_out``
-    with the module's ``row_tile`` / ``groups_per_split`` and arithmetic (the
-    table kernel, fp32 split partials summed in split order), one preallocated
-    workspace.  Serves ``decoded_bf16`` and any ``groups_per_split > 1``."""
+    with the module's ``row_tile`` / ``groups_per_split`` and arithmetic (fp32 split
+    partials summed in split order), one preallocated workspace.  Serves ``decoded_bf16`` and any ``groups_per_split > 1``."""
 
     def __init__(self, module: "PackedW3Linear", device: torch.device):
         self.module = module
@@ -407,7 +409,9 @@ class PackedW3Linear(PackedLinearBase):
     and the reference's table contract (``w3_lut_m1_out``: ``row_tile``,
     ``groups_per_split``, split partials summed in order) for routes that split K,
     as ``observed_exact`` does at the gate/up and down shapes.  The dense fallback
-    dequantizes with the HIP restore kernel on GPU.
+    on GPU is the HIP GEMM on the payload up to ``GEMM_MAX_ROWS`` rows, and the HIP
+    restore kernel with ``F.linear`` for more rows and for the inputs that the GEMM
+    does not take.
 
     ``max_packed_rows`` (not in the reference; default 1) lets 2..8-row inputs
     take the MFMA kernel too; they are then counted under ``packed_small_m``.
