@@ -225,7 +225,7 @@ class _Restored:
         g, o = codes.shape[:2]
         device = codes.device
         self.weight = torch.empty((o, g * GROUP), dtype=dtype, device=device)
-        self._bad = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self._bad = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
         _lib.check(_lib.library().fx_hybrid_restore(
             codes.data_ptr(), p["rows"].data_ptr(), p["columns"].data_ptr(), p["indices"].data_ptr(),
             p["sparse_codes"].data_ptr(), p["sparse_rows"].data_ptr(), p["sparse_columns"].data_ptr(),

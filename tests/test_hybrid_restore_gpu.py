@@ -45,3 +45,11 @@ def test_restore_refuses_what_torch_refuses(gpu, field, where, value, message):
         module(x)
     with pytest.raises(ValueError, match=message):
         d.decode_layout(module.layout())
+
+
+def test_restore_under_a_default_device(gpu):
+    """The verdict lives in pinned host memory whatever device new tensors go to."""
+    layout = _layout(17, 3, "v5_p1024", gpu)
+    want = d._decode_layout_torch(layout, torch.bfloat16)
+    with torch.device(gpu):
+        assert torch.equal(d.decode_layout(layout), want)
