@@ -38,7 +38,7 @@ from torch.nn import functional as F
 
 from . import _lib
 from .evaluation import materialize_hybrid_s8_weight, tensor_sha256
-from .packed_linear import PackedLinearBase, replace_linears_atomically
+from .packed_linear import PackedLinearBase, replace_linears_atomically, untraced
 
 FORMAT = "fluxbin-hybrid-g128-s8-m1-v1"
 PLANAR_FORMAT = "fluxbin-hybrid-g128-s8-m1-planar-v1"
@@ -197,10 +197,10 @@ _RESTORE_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 
 def _restore_kernel_takes(p: Mapping[str, torch.Tensor], dtype) -> bool:
     """The layouts ``fx_hybrid_restore`` reads: one GPU, contiguous fields of the
-    types and shapes ``convert_artifact`` writes, aligned to their elements' pairs.
-    The torch arithmetic takes (or refuses) every other one."""
+    types and shapes ``convert_artifact`` writes, aligned to their elements' pairs,
+    and no tracer that would record the weight without its values.  The torch arithmetic takes (or refuses) every other one."""
     codes = p["codes"]
-    if not codes.is_cuda or dtype not in _RESTORE_DTYPES or torch.cuda.is_current_stream_capturing():
+    if not codes.is_cuda or not untraced() or dtype not in _RESTORE_DTYPES or torch.cuda.is_current_stream_capturing():
         return False
     g, o = codes.shape[0], codes.shape[1] if codes.ndim > 1 else 0
     planar = codes.ndim == 4

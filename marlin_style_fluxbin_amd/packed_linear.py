@@ -36,14 +36,20 @@ PACKED_M1, DENSE_FALLBACK, PACKED_SMALL_M = "packed_m1", "dense_fallback", "pack
 PackedKernel = Callable[[torch.Tensor, torch.Tensor], torch.Tensor]  # (x [rows, K], out [rows, O]) -> out
 
 
+def untraced() -> bool:
+    """True when no tracer or dispatch mode records the torch ops of this call: what a
+    kernel called by address writes would be missing from such a record."""
+    return (not torch.compiler.is_compiling() and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._get_tracing_state() is None)
+
+
 def plain_call(x: torch.Tensor) -> bool:
     """True when a kernel called by address computes what a torch op on ``x`` would:
     a plain tensor, and no tracer, dispatch or function mode, transform (vmap, jvp)
     or autocast in force that has to see (or would change) the op."""
-    return (type(x) is torch.Tensor and not torch.is_autocast_enabled("cuda")
-            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
-            and torch._C._functorch.maybe_current_level() is None and forward_ad._current_level < 0
-            and torch._C._get_tracing_state() is None)
+    return (untraced() and type(x) is torch.Tensor and not torch.is_autocast_enabled("cuda")
+            and torch._C._len_torch_function_stack() == 0
+            and torch._C._functorch.maybe_current_level() is None and forward_ad._current_level < 0)
 
 
 class PackedLinearBase(nn.Module):

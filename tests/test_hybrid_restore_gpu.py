@@ -3,6 +3,7 @@ arithmetic it replaces on the GPU: bitwise in every output type and both code
 formats at row counts off the workgroup's 128 and 16, and the same refusals."""
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from marlin_style_fluxbin_amd import deployment as d
 from oracle import two_base as tb
@@ -53,3 +54,22 @@ def test_restore_under_a_default_device(gpu):
     want = d._decode_layout_torch(layout, torch.bfloat16)
     with torch.device(gpu):
         assert torch.equal(d.decode_layout(layout), want)
+
+
+class _Seen(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def test_traced_calls_keep_the_torch_arithmetic(gpu):
+    """A tracer records torch ops: the weight has to be formed by them."""
+    p = {k: torch.from_numpy(v) for k, v in tb.make_hybrid_payload(48, 2, seed=5).items()}
+    module = d.PackedHybridLinear(p, fallback="dense", kernel="v5_p1024").to(gpu)
+    x = torch.randn(3, 256, device=gpu).to(torch.bfloat16)
+    with _Seen():
+        assert not d._restore_kernel_takes(module.layout(), torch.bfloat16)
+    with torch.no_grad():
+        want = module(x)
+        traced = torch.jit.trace(module, x, check_trace=False)
+        assert "aten::empty(" not in str(traced.inlined_graph.findNode("aten::linear").inputsAt(1).node())
+        assert torch.equal(traced(x), want)
