@@ -178,7 +178,7 @@ class PackedLinearBase(nn.Module):
         flat = len(shape) == 2
         out = torch.empty((rows, o), device=device, dtype=x.dtype)
         self._packed_kernel(rows, device)((x if flat else x.reshape(rows, k)).contiguous(), out)
-        bias = self._buffers["bias"]
+        bias = self.bias
         if bias is not None:
             out = out.add_(bias) if self.bias_in_place else out + bias
         return out if flat else out.reshape(*shape[:-1], o)

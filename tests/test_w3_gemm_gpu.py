@@ -107,3 +107,17 @@ def test_gemm_route_leaves_other_calls_alone(gpu):
     assert not mixed._gemm_takes(x)
     with torch.inference_mode(), pytest.raises(RuntimeError):
         mixed(x)
+
+
+def test_gemm_takes_only_whole_biases(gpu):
+    """A bias that F.linear would broadcast keeps F.linear; one held as a Parameter is read."""
+    x = torch.randn(20, 256, device=gpu).to(torch.bfloat16)
+    one = _module(gpu, 64, 256, bias=torch.ones(1, device=gpu, dtype=torch.bfloat16))
+    assert not one._gemm_takes(x)
+    whole = _module(gpu, 64, 256, bias=torch.zeros(64, device=gpu, dtype=torch.bfloat16))
+    whole.bias = torch.nn.Parameter(torch.ones(64, device=gpu, dtype=torch.bfloat16), requires_grad=False)
+    _check(whole, x, "bf16")
+    with torch.inference_mode():
+        want = torch.nn.functional.linear(x, one._dense_weight(torch.bfloat16), one.bias)
+        assert torch.equal(one(x), want)
+        assert torch.equal(_module(gpu, 64, 256, bias=whole.bias, max_packed_rows=1)(x[:1]), whole(x[:1]))

@@ -290,3 +290,13 @@ def test_route_counter_reset_keeps_the_small_m_key():
     assert validate_routes(trace, expected_linears=2, steps=1)
     trace["routes"]["a"]["dense_fallback"] = 1  # the prompt served twice
     assert not validate_routes(trace, expected_linears=2, steps=1)
+
+
+def test_module_takes_a_bias_parameter():
+    """Assigning a Parameter moves ``bias`` from the module's buffers to its parameters."""
+    module = wl.PackedW3Linear(tiny_layout(), bias=torch.zeros(32), fallback="dense", row_tile=256)
+    bias = torch.randn(32, generator=torch.Generator().manual_seed(1))
+    module.bias = nn.Parameter(bias, requires_grad=False)
+    x = torch.randn(3, 128, generator=torch.Generator().manual_seed(2))
+    with torch.inference_mode():
+        assert torch.equal(module(x), nn.functional.linear(x, module._dense_weight(x.dtype), bias))
