@@ -45,9 +45,10 @@ def untraced() -> bool:
 
 def plain_call(x: torch.Tensor) -> bool:
     """True when a kernel called by address computes what a torch op on ``x`` would:
-    a plain tensor, and no tracer, dispatch or function mode, transform (vmap, jvp)
-    or autocast in force that has to see (or would change) the op."""
-    return (untraced() and type(x) is torch.Tensor and not torch.is_autocast_enabled("cuda")
+    a plain tensor that holds its own values (no lazy negation), and no tracer, dispatch
+    or function mode, transform (vmap, jvp) or autocast in force that has to see (or
+    would change) the op."""
+    return (untraced() and type(x) is torch.Tensor and not x.is_neg() and not torch.is_autocast_enabled("cuda")
             and torch._C._len_torch_function_stack() == 0
             and torch._C._functorch.maybe_current_level() is None and forward_ad._current_level < 0)
 

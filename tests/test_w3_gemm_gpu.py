@@ -121,3 +121,15 @@ def test_gemm_takes_only_whole_biases(gpu):
         want = torch.nn.functional.linear(x, one._dense_weight(torch.bfloat16), one.bias)
         assert torch.equal(one(x), want)
         assert torch.equal(_module(gpu, 64, 256, bias=whole.bias, max_packed_rows=1)(x[:1]), whole(x[:1]))
+
+
+def test_gemm_leaves_lazy_negation_to_torch(gpu):
+    """A conjugate's imaginary part is a view whose memory holds the other sign."""
+    module = _module(gpu, 64, 256, scale="f16")
+    x = torch.zeros(20, 256, dtype=torch.complex32, device=gpu)
+    x.copy_(torch.randn(20, 256, dtype=torch.complex64, device=gpu))
+    lazy = x.conj().imag
+    assert lazy.is_neg() and not module._gemm_takes(lazy)
+    with torch.inference_mode():
+        want = torch.nn.functional.linear(lazy, module._dense_weight(torch.float16))
+        assert torch.equal(module(lazy), want)
