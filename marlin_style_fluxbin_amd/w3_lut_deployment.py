@@ -469,10 +469,10 @@ class PackedW3Linear(PackedLinearBase):
     def _gemm_takes(self, x: torch.Tensor) -> bool:
         """The dense-fallback inputs that ``fx_w3_gemm`` multiplies; the restored
         weight and ``F.linear`` take (or refuse) every other one."""
-        planes, bias = self.planes, self.bias
+        planes, bias = self._tensor("planes"), self._tensor("bias")
         return (x.is_cuda and x.dtype in HALF_DTYPES and x.device == planes.device and plain_call(x)
                 and 0 < x.numel() <= GEMM_MAX_ROWS * self.in_features
-                and planes.numel() < 2**31 and planes.data_ptr() % 16 == 0 and self.perm.data_ptr() % 16 == 0
+                and planes.numel() < 2**31 and planes.data_ptr() % 16 == 0 and self._tensor("perm").data_ptr() % 16 == 0
                 and (bias is None or (bias.dtype == x.dtype and bias.device == x.device and bias.is_contiguous()
                                       and bias.shape == (self.out_features,))))
 
@@ -500,7 +500,7 @@ class PackedW3Linear(PackedLinearBase):
         rc = lib.fx_w3_gemm(
             x.data_ptr(), _lib.dtype_code(dtype), layout["planes"].data_ptr(), scales.data_ptr(),
             _lib.dtype_code(scales.dtype), _lib.ptr(layout.get("zeros")),
-            None if self._perm_identity else layout["perm"].data_ptr(), _lib.ptr(self.bias),
+            None if self._perm_identity else layout["perm"].data_ptr(), _lib.ptr(self._tensor("bias")),
             workspace.data_ptr(), nbytes, out.data_ptr(), rows, o, k, _lib.stream_handle(device))
         if rc:
             _lib.check(rc, "fx_w3_gemm")
@@ -518,7 +518,7 @@ class PackedW3Linear(PackedLinearBase):
             if self._table is None or self._table.workspace.device != device:
                 self._table = _TableRoute(self, device)
             return self._table
-        if self._gemv is None or self._gemv.layout["planes"].data_ptr() != self.planes.data_ptr():
+        if self._gemv is None or self._gemv.layout["planes"].data_ptr() != self._tensor("planes").data_ptr():
             self._gemv = W3Gemv(self.layout(), arithmetic=self.arithmetic, perm_identity=self._perm_identity,
                                 max_rows=self.max_packed_rows)
         return self._gemv
