@@ -38,7 +38,8 @@ from torch.nn import functional as F
 
 from . import _lib
 from .evaluation import materialize_hybrid_s8_weight, tensor_sha256
-from .packed_linear import PackedLinearBase, replace_linears_atomically, untraced
+from .packed_linear import (
+    PackedLinearBase, holds_values, only_default_device, replace_linears_atomically, untraced, untransformed)
 
 FORMAT = "fluxbin-hybrid-g128-s8-m1-v1"
 PLANAR_FORMAT = "fluxbin-hybrid-g128-s8-m1-planar-v1"
@@ -197,10 +198,13 @@ _RESTORE_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 
 def _restore_kernel_takes(p: Mapping[str, torch.Tensor], dtype) -> bool:
     """The layouts ``fx_hybrid_restore`` reads: one GPU, contiguous fields of the
-    types and shapes ``convert_artifact`` writes, aligned to their elements' pairs,
-    and no tracer that would record the weight without its values.  The torch arithmetic takes (or refuses) every other one."""
+    types and shapes ``convert_artifact`` writes that hold their values in memory, aligned
+    to their elements' pairs, and nothing in force that has to see the weight formed: a
+    tracer or mode, a transform, a graph through a field.  The torch arithmetic takes (or
+    refuses) every other one."""
     codes = p["codes"]
-    if not codes.is_cuda or not untraced() or dtype not in _RESTORE_DTYPES or torch.cuda.is_current_stream_capturing():
+    if (not codes.is_cuda or not untraced() or not untransformed() or not only_default_device()
+            or dtype not in _RESTORE_DTYPES or torch.cuda.is_current_stream_capturing()):
         return False
     g, o = codes.shape[0], codes.shape[1] if codes.ndim > 1 else 0
     planar = codes.ndim == 4
@@ -210,8 +214,13 @@ def _restore_kernel_takes(p: Mapping[str, torch.Tensor], dtype) -> bool:
     types = {"codes": torch.uint8, "sparse_codes": torch.uint8, "indices": torch.int16}
     if not (1 <= o <= 65536 and 1 <= g <= 1024):
         return False
-    return all(p[n].shape == s and p[n].dtype == types.get(n, torch.float32) and p[n].device == codes.device
-               and p[n].is_contiguous() and p[n].data_ptr() % 8 == 0 for n, s in shapes.items())
+    device, recording = codes.device, torch.is_grad_enabled()
+    for name, shape in shapes.items():
+        t = p[name]
+        if (t.shape != shape or t.dtype != types.get(name, torch.float32) or t.device != device
+                or not holds_values(t, recording) or not t.is_contiguous() or t.data_ptr() % 8 != 0):
+            return False
+    return True
 
 
 class _Restored:

@@ -29,10 +29,13 @@ import torch
 from torch import nn
 from torch.autograd import forward_ad
 from torch.nn import functional as F
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 HALF_DTYPES = (torch.float16, torch.bfloat16)
 PACKED_M1, DENSE_FALLBACK, PACKED_SMALL_M = "packed_m1", "dense_fallback", "packed_small_m"
 
+_PLAIN_TYPES = (torch.Tensor, nn.Parameter)
 PackedKernel = Callable[[torch.Tensor, torch.Tensor], torch.Tensor]  # (x [rows, K], out [rows, O]) -> out
 
 
@@ -43,14 +46,32 @@ def untraced() -> bool:
             and torch._C._get_tracing_state() is None)
 
 
+def untransformed() -> bool:
+    """True when no transform (vmap, jvp, grad) and no forward-mode level is in force: what
+    a kernel called by address writes carries neither a batch dimension nor a tangent."""
+    return torch._C._functorch.maybe_current_level() is None and forward_ad._current_level < 0
+
+
+def only_default_device() -> bool:
+    """True when no torch function mode but torch's own default-device context (which
+    changes factory calls alone) is in force."""
+    return torch._C._len_torch_function_stack() == 0 or all(
+        type(mode) is DeviceContext for mode in _get_current_function_mode_stack())
+
+
+def holds_values(t: torch.Tensor, recording: bool) -> bool:
+    """True when ``t``'s memory holds its values (no subclass, no lazy negation) and no
+    graph is recorded through it (``recording``: grad mode is on)."""
+    return type(t) in _PLAIN_TYPES and not t.is_neg() and not (recording and t.requires_grad)
+
+
 def plain_call(x: torch.Tensor) -> bool:
     """True when a kernel called by address computes what a torch op on ``x`` would:
     a plain tensor that holds its own values (no lazy negation), and no tracer, dispatch
     or function mode, transform (vmap, jvp) or autocast in force that has to see (or
     would change) the op."""
     return (untraced() and type(x) is torch.Tensor and not x.is_neg() and not torch.is_autocast_enabled("cuda")
-            and torch._C._len_torch_function_stack() == 0
-            and torch._C._functorch.maybe_current_level() is None and forward_ad._current_level < 0)
+            and torch._C._len_torch_function_stack() == 0 and untransformed())
 
 
 class PackedLinearBase(nn.Module):

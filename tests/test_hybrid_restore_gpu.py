@@ -3,6 +3,8 @@ arithmetic it replaces on the GPU: bitwise in every output type and both code
 formats at row counts off the workgroup's 128 and 16, and the same refusals."""
 import pytest
 import torch
+from torch.autograd import forward_ad
+from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
 from marlin_style_fluxbin_amd import deployment as d
@@ -73,3 +75,69 @@ def test_traced_calls_keep_the_torch_arithmetic(gpu):
         traced = torch.jit.trace(module, x, check_trace=False)
         assert "aten::empty(" not in str(traced.inlined_graph.findNode("aten::linear").inputsAt(1).node())
         assert torch.equal(traced(x), want)
+
+
+def _module(gpu, o=48, g=2):
+    p = {k: torch.from_numpy(v) for k, v in tb.make_hybrid_payload(o, g, seed=5).items()}
+    return d.PackedHybridLinear(p, fallback="dense", kernel="v5_p1024").to(gpu)
+
+
+@pytest.mark.parametrize("field", ["rows", "columns", "sparse_rows", "sparse_columns"])
+def test_restored_weight_keeps_derivatives(gpu, field):
+    """Scales with a gradient or a tangent: the weight is a function of them."""
+    layout = _layout(33, 2, "v5_p1024", gpu)
+    head = torch.randn(33, 256, generator=torch.Generator().manual_seed(1)).to(gpu)
+
+    def gradient(decode):
+        leaf = layout[field].clone().requires_grad_()
+        return torch.autograd.grad((decode(dict(layout, **{field: leaf}), torch.float32) * head).sum(), leaf)[0]
+
+    want = gradient(d._decode_layout_torch)
+    assert bool(want.any()) and torch.equal(gradient(d.decode_layout), want)
+    leaf = layout[field].clone().requires_grad_()
+    with torch.no_grad():  # no graph is asked for: the kernel may form the values
+        assert torch.equal(d.decode_layout(dict(layout, **{field: leaf})), d.decode_layout(layout))
+    tangent = torch.randn(layout[field].shape, generator=torch.Generator().manual_seed(2)).to(gpu)
+    with torch.no_grad(), forward_ad.dual_level():
+        dual = dict(layout, **{field: forward_ad.make_dual(layout[field], tangent)})
+        got = forward_ad.unpack_dual(d.decode_layout(dual, torch.float32)).tangent
+        want = forward_ad.unpack_dual(d._decode_layout_torch(dual, torch.float32)).tangent
+    assert got is not None and torch.equal(got, want)
+
+
+def test_transforms_over_the_module(gpu):
+    module = _module(gpu)
+    x, t = (torch.randn(3, 256, generator=torch.Generator().manual_seed(i)).to(torch.bfloat16).to(gpu) for i in (0, 1))
+    w = d._decode_layout_torch(module.layout(), torch.bfloat16)
+    with torch.no_grad():
+        y, dy = torch.func.jvp(module, (x,), (t,))
+        assert torch.equal(y, torch.nn.functional.linear(x, w)) and torch.equal(dy, torch.nn.functional.linear(t, w))
+        assert torch.equal(torch.func.vmap(module)(x.view(1, 3, 256))[0], y)
+
+
+def test_restore_leaves_lazy_negation_to_torch(gpu):
+    """A contiguous view whose memory holds the other sign."""
+    layout = _layout(17, 3, "v5_p1024", gpu)
+    want = d.decode_layout(layout)
+    for field in ("rows", "columns", "sparse_rows", "sparse_columns"):
+        lazy = torch._neg_view(-layout[field])
+        assert lazy.is_neg() and lazy.is_contiguous()
+        assert torch.equal(d.decode_layout(dict(layout, **{field: lazy})), want)
+
+
+class _Doubled(TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        out = func(*args, **(kwargs or {}))
+        return out.mul_(2) if func is torch.Tensor.scatter_add_ else out
+
+
+def test_function_modes_see_the_torch_arithmetic(gpu):
+    """A function mode may change any op of the dequantize; torch's default device is
+    one that changes none."""
+    layout = _layout(17, 3, "v5_p1024", gpu)
+    with _Doubled():
+        assert not d._restore_kernel_takes(layout, torch.bfloat16)
+        doubled = d.decode_layout(layout, torch.float32)
+    assert torch.equal(doubled, 2 * d._decode_layout_torch(layout, torch.float32))
+    with torch.device(gpu):
+        assert d._restore_kernel_takes(layout, torch.bfloat16)
