@@ -177,6 +177,15 @@ __device__ __forceinline__ int lane_times_rows(int lane_index, int rows) {
 // guards that convergent cross-lane operations cannot follow.
 __device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6); }
 
+// Between a wave's LDS writes and other lanes' reads of them.  The hardware runs a wave's
+// LDS operations in order; the fences say so to the compiler, which sees each lane's own
+// accesses only (a scheduling barrier alone is no memory fence).  No instruction.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Sum over the 64 lanes of a wave (DPP within rows of 16, then lanes 16 and 32
 // apart); every lane gets the same bits.
 __device__ __forceinline__ float wave_total(float v) {

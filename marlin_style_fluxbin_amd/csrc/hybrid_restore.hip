@@ -56,8 +56,9 @@ __device__ __forceinline__ float two_base(unsigned s0, unsigned s1, const float2
 template <int WDT>
 __global__ __launch_bounds__(256) void hybrid_restore_kernel(HybridRestoreArgs a) {
   using Element = std::conditional_t<WDT == kF32, float, uint16_t>;
+  typedef Element __attribute__((may_alias)) StagedElement;  // one value of a staged vector
   constexpr int kVecs = 8 * int(sizeof(Element)) / 16;  // 16-byte vectors of 8 columns
-  __shared__ uint4 stage[4][8][16 * kVecs];
+  __shared__ u32x4_t stage[4][8][16 * kVecs];
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int c = lane & 15;
   const int g = int(blockIdx.x % unsigned(a.G));
@@ -122,15 +123,15 @@ __global__ __launch_bounds__(256) void hybrid_restore_kernel(HybridRestoreArgs a
       float v[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = two_base((p0 >> e) & 1u, (p1 >> e) & 1u, in.row[h], col[e][0], col[e][1]);
-      uint4* dst = &stage[wave][4 * h + (lane >> 4)][c * kVecs];
+      u32x4_t* dst = &stage[wave][4 * h + (lane >> 4)][c * kVecs];
       if constexpr (WDT == kF32) {
-        dst[0] = make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3]));
-        dst[1] = make_uint4(__float_as_uint(v[4]), __float_as_uint(v[5]), __float_as_uint(v[6]), __float_as_uint(v[7]));
+        dst[0] = u32x4_t{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+        dst[1] = u32x4_t{__float_as_uint(v[4]), __float_as_uint(v[5]), __float_as_uint(v[6]), __float_as_uint(v[7])};
       } else {
         unsigned pair[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) pair[e] = round_pair_bits<WDT>(v[2 * e], v[2 * e + 1]);
-        dst[0] = make_uint4(pair[0], pair[1], pair[2], pair[3]);
+        dst[0] = u32x4_t{pair[0], pair[1], pair[2], pair[3]};
       }
     }
     {
@@ -138,22 +139,22 @@ __global__ __launch_bounds__(256) void hybrid_restore_kernel(HybridRestoreArgs a
       bad |= not_finite(in.srow.x) || not_finite(in.srow.y);
       const float w = two_base((p0 >> (at & 7)) & 1u, (p1 >> (at & 7)) & 1u, in.prow, rcol.x, rcol.y) +
                       two_base((q0 >> slot) & 1u, (q1 >> slot) & 1u, in.srow, ucol.x, ucol.y);
-      __builtin_amdgcn_wave_barrier();  // after the row's own values (LDS operations of a wave run in order)
-      Element* dst = reinterpret_cast<Element*>(&stage[wave][lane >> 3][0]) + at;
+      wave_lds_order();  // after the row's own values
+      StagedElement* dst = reinterpret_cast<StagedElement*>(&stage[wave][lane >> 3][0]) + at;
       if constexpr (WDT == kF32) *dst = w;
       else *dst = from_f32<WDT>(w);
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_order();
     }
 #pragma unroll
     for (int n = 0; n < 2 * kVecs; ++n) {
       const int unit = n * 64 + lane, rr = unit / (16 * kVecs), at16 = unit % (16 * kVecs);
-      const uint4 v = stage[wave][rr][at16];
+      const u32x4_t v = stage[wave][rr][at16];
       const int o = i + rr;
       if (o < a.O)
-        *reinterpret_cast<uint4*>(static_cast<Element*>(a.weight) + size_t(o) * (size_t(a.G) * 128) + size_t(g) * 128 +
+        *reinterpret_cast<u32x4_t*>(static_cast<Element*>(a.weight) + size_t(o) * (size_t(a.G) * 128) + size_t(g) * 128 +
                                   at16 * (16 / int(sizeof(Element)))) = v;
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_order();
   }
   if (bad) *a.bad = 1;  // every writer stores the same value
 }

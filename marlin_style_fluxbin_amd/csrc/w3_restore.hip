@@ -62,7 +62,7 @@ __global__ __launch_bounds__(256) void w3_restore_kernel(RestoreArgs a) {
 #pragma unroll
     for (int b = 0; b < 4; ++b) stage[wave][r * (kRow + 1) + i * 16 + b * 4 + w] = v[b];  // vector 4 w + b of the group
   }
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_order();
   const size_t K = size_t(a.G) * 128;
 #pragma unroll
   for (int k = 0; k < 16 * kRow / 64; ++k) {
