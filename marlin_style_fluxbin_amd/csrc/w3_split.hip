@@ -11,12 +11,20 @@
 // one-split launches: 315 -> 110 us).  The bound is the chain of loads, gather and
 // expansion of six waves a SIMD (with 92 registers, five waves: 11.2).
 //
-// Weights.  s (q - z) is a 16-bit number at most (bf16 or fp16 scale times a small
-// integer), so it is exactly hi + lo of two bf16 values; decoded_bf16 arithmetic drops
-// lo where |q - z| = 3, which is all it needs when every zero-point is 3 or 4 (the other
-// products are bf16 numbers): the lo chain runs only for structural arithmetic or where
-// a lane sees another zero-point.  fp16 activations are split the same way into two
-// columns.  Every product is exact in fp32.
+// Weights.  With a zero-point of 0..7, s (q - z) has at most 14 significant bits (bf16 or
+// fp16 scale times an integer of three bits), so it is exactly hi + lo of two bf16 values;
+// decoded_bf16 arithmetic drops lo where |q - z| = 3, which is all it needs when every
+// zero-point is 3 or 4 (the other products are bf16 numbers): the lo chain runs only for
+// structural arithmetic or where a lane sees another zero-point.  fp16 activations are
+// split the same way into two columns.  Every product is exact in fp32.
+//
+// Zero-points above 7 (the entry points take the whole byte; a checked layout has none)
+// need up to 19 bits, and a scale that is not finite, or whose products overflow bf16,
+// would reach the other splits of its batch as 0 x infinity.  Where a batch holds such a
+// (row, group), the row's sums are formed again in fp32, in the table kernel's arithmetic
+// (odd_group), after the matrix chain.  The others pay a compare a batch for it: two
+// layers' Linears on the observed_exact route take 110.0 us with it and 109.4 without
+// (111 with the odd weights' tables zeroed ahead of the chain and their sums added).
 //
 // A workgroup owns 16 rows; wave w takes the four-group batches w, w + 8, ...  k-block
 // l / 16 of an instruction carries group 4 i + l / 16, and column 2 j (+ 1 for the low
@@ -57,6 +65,44 @@ __device__ __forceinline__ unsigned finite_pair(unsigned v) {
   return lo | ((v & 0x7f800000u) == 0x7f800000u ? 0u : v & 0xffff0000u);
 }
 
+// Whether a (row, group)'s weights are not each two bf16 values: |q - z| > 7, or |s| of
+// 2^125 and more (bf16: 7 s overflows), infinite or NaN.
+__device__ __forceinline__ bool is_odd_group(unsigned scale_bits, unsigned zero, int sdt) {
+  return zero > 7u || (scale_bits & 0x7fffu) >= (sdt == kBF16 ? 0x7e00u : 0x7c00u);
+}
+
+// One (row, group)'s sum in fp32: s sum (q - z) x, and for decoded arithmetic the
+// correction of the weights with |q - z| = 3.  planes: its 16 bytes a plane, from `at` on;
+// x: the group's 16 operand units (their low digits `low_units` on, with fp16
+// activations).  Rare and small rather than fast: one byte column at a time.
+template <int XDT>
+__device__ __forceinline__ float odd_group(__amdgpu_buffer_rsrc_t planes, int at, int plane_stride, const u32x4_t* x,
+                                           int low_units, unsigned scale_bits, unsigned zero, int sdt, bool decoded) {
+  float dot = 0.f, three = 0.f;
+#pragma unroll 1
+  for (int c = 0; c < 16; ++c) {
+    const u32x4_t hi = x[c];
+    u32x4_t lo = {0u, 0u, 0u, 0u};
+    if constexpr (XDT == kF16) lo = x[low_units + c];
+    unsigned b[3];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) b[p] = __builtin_amdgcn_raw_buffer_load_b8(planes, at + c, p * plane_stride, 0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int shift = 16 * (j & 1);
+      const float v = to_f32<kBF16>(uint16_t(hi[j >> 1] >> shift)) + to_f32<kBF16>(uint16_t(lo[j >> 1] >> shift));
+      const int q = int(((b[0] >> j) & 1u) | (((b[1] >> j) & 1u) << 1) | (((~b[2] >> j) & 1u) << 2)), d = q - int(zero);
+      dot += float(d) * v;
+      if (d == 3) three += v;
+      if (d == -3) three -= v;
+    }
+  }
+  const float s = sdt == kBF16 ? to_f32<kBF16>(uint16_t(scale_bits)) : to_f32<kF16>(uint16_t(scale_bits));
+  float sum = dot * s;
+  if (decoded) sum += three * (round_to<kBF16>(3.f * s) - 3.f * s);
+  return sum;
+}
+
 // Elements 8 i .. 8 i + 7 of a 16-bit array.
 __device__ __forceinline__ u32x4_t load_eight(const uint16_t* p, int i, int aligned) {
   if (aligned) return reinterpret_cast<const u32x4_t*>(p)[i];
@@ -82,7 +128,7 @@ __global__ __launch_bounds__(kSplitWaves * 64, 6) void w3_split_kernel(SplitArgs
   u32x4_t* xs = split_lds;
   u32x4_t* zero16 = xs + kDigits * units;
   float* sums = reinterpret_cast<float*>(zero16 + 16);
-  const int slots = a.gps < 4 && a.gps < a.G ? 4 / a.gps : 1;  // splits in a batch
+  const int slots = 4 >> a.slot_shift;  // splits in a batch
   uint16_t* raw = reinterpret_cast<uint16_t*>(sums + batches * slots * 16);
 
   // ---- activations and their columns first (the wave's loads complete in order, and
@@ -107,10 +153,11 @@ __global__ __launch_bounds__(kSplitWaves * 64, 6) void w3_split_kernel(SplitArgs
     u32x4_t p[3];
     unsigned s, z;
   };
+  const auto plane_offset = [&](int batch) { return (4 * batch * 3 * a.O + lane_times_rows(kb, 3 * a.O) + row) * 16; };
   auto issue = [&](int batch, Loads& L) __attribute__((always_inline)) {
     const int out = batch < batches && 4 * batch + kb < a.G ? 0 : kOutOfRange;  // zero scales: zero weights
     const int e = 4 * batch * a.O + lane_times_rows(kb, a.O) + row;
-    const int off = ((4 * batch * 3 * a.O + lane_times_rows(kb, 3 * a.O) + row) * 16) | out;
+    const int off = plane_offset(batch) | out;
     L.s = __builtin_amdgcn_raw_buffer_load_b16(rs, (e * 2) | out, 0, 0);
     L.z = __builtin_amdgcn_raw_buffer_load_b8(rz, e | out, 0, 0);
 #pragma unroll
@@ -165,13 +212,15 @@ __global__ __launch_bounds__(kSplitWaves * 64, 6) void w3_split_kernel(SplitArgs
   __syncthreads();
 
   // ---- this lane's operand: column c = 2 slot + digit, its own split's groups
-  const int slot = slots == 1 ? 0 : kb / a.gps;
+  const int slot = kb >> a.slot_shift;
   const int digit = c & 1;
   const bool active = (c >> 1) == slot && digit < kDigits;
+  unsigned long long any_odd = 0;  // lanes with an odd group in one of the wave's batches
   for (int batch = wave; batch < batches; batch += kSplitWaves) {
     const Loads cur = next;
     issue(batch + kSplitWaves, next);
     const unsigned zero = (cur.z & 0xffu) | zero_default;
+    any_odd |= __builtin_amdgcn_ballot_w64(is_odd_group(cur.s, zero, a.sdt));
     ValueTable hi, lo;
     split_tables(cur.s, zero, a.sdt, a.decoded, hi, lo);
     const bool low = !a.decoded || __builtin_amdgcn_ballot_w64(zero != 3u && zero != 4u && 4 * batch + kb < a.G) != 0;
@@ -215,6 +264,24 @@ __global__ __launch_bounds__(kSplitWaves * 64, 6) void w3_split_kernel(SplitArgs
       for (int j = 0; j < 4; ++j) sums[(batch * slots + (c >> 1)) * 16 + 4 * kb + j] = d[j];
     }
   }
+  // ---- odd groups: the sums of their rows in their batches, formed again
+  for (int batch = wave; any_odd != 0 && batch < batches; batch += kSplitWaves) {
+    Loads L;
+    issue(batch, L);
+    const unsigned zero = (L.z & 0xffu) | zero_default;
+    const unsigned long long odd = __builtin_amdgcn_ballot_w64(is_odd_group(L.s, zero, a.sdt));
+    if (((odd | odd >> 16 | odd >> 32 | odd >> 48) >> r) & 1u) {  // this lane's row has one
+      float sum = 0.f;
+      if (4 * batch + kb < a.G)
+        sum = odd_group<XDT>(rp, plane_offset(batch), a.O * 16, xs + batch * 64 + kb * 16, units, L.s, zero, a.sdt, a.decoded);
+      float* at = sums + (batch * slots + slot) * 16 + r;
+#pragma unroll 1
+      for (int k = 0; k < 4; ++k) {  // the groups in turn; a split's first one starts its sum
+        wave_lds_order();
+        if (kb == k) *at = k == slot << a.slot_shift ? sum : *at + sum;
+      }
+    }
+  }
   __syncthreads();
 
   // ---- partials in batch order (over the batches' sums), the output in split order;
@@ -255,8 +322,9 @@ __global__ __launch_bounds__(kSplitWaves * 64, 6) void w3_split_kernel(SplitArgs
   if (a.out && threadIdx.x < 16 && o < a.O) a.out[o] = from_f32<XDT>(total(0, splits));
 }
 
-void launch_split(int xdt, const SplitArgs& a, hipStream_t s) {
-  const int batches = (a.G + 3) / 4, slots = a.gps < 4 && a.gps < a.G ? 4 / a.gps : 1;
+void launch_split(int xdt, SplitArgs a, hipStream_t s) {
+  a.slot_shift = a.gps >= 4 || a.gps >= a.G ? 2 : a.gps - 1;
+  const int batches = (a.G + 3) / 4, slots = 4 >> a.slot_shift;
   const size_t lds = size_t(batches) * 1024 * (xdt == kF16 ? 2 : 1) + 256 + size_t(batches) * slots * 64 +
                      (a.perm ? size_t(a.G) * 256 : 0);
   const dim3 grid(unsigned((a.O + 15) / 16)), block(kSplitWaves * 64);

@@ -19,6 +19,7 @@ struct SplitArgs {
   int sdt;      // scale dtype
   int decoded;  // weights with |q - z| = 3 rounded to bf16
   int x16, perm16;  // 16-byte aligned
+  int slot_shift;   // log2 of the groups of a batch in one split (launch_split sets it)
 };
 
 constexpr int kSplitMaxColumns = 16384;
@@ -27,6 +28,6 @@ constexpr int kSplitMaxColumns = 16384;
 inline bool split_kernel_takes(int G, int gps) {
   return G * 128 <= kSplitMaxColumns && (gps >= G || gps % 4 == 0 || gps == 1 || gps == 2);
 }
-void launch_split(int xdt, const SplitArgs& a, hipStream_t s);
+void launch_split(int xdt, SplitArgs a, hipStream_t s);
 
 }  // namespace fx

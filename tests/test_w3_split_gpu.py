@@ -86,3 +86,69 @@ def test_split_infinities(gpu, dtype):
     assert torch.equal(torch.isnan(partial), torch.isnan(want))
     finite_sign = ~torch.isnan(want)
     assert torch.equal(partial[finite_sign], want[finite_sign].float())
+
+
+def _partials(layout, x, gps, decoded, row_tile=256):
+    g, _, o, _ = layout["planes"].shape
+    partial = torch.full((-(-g // gps), o), float("nan"), device=x.device)
+    _lib.check(_lib.library().fx_w3_inline_main(
+        x.data_ptr(), _lib.dtype_code(x.dtype), layout["planes"].data_ptr(), layout["scales"].data_ptr(),
+        _lib.dtype_code(layout["scales"].dtype), layout["zeros"].data_ptr(), layout["perm"].data_ptr(),
+        partial.data_ptr(), 1, o, 128 * g, gps, row_tile, int(decoded), _lib.stream_handle(x.device)), "main")
+    return partial
+
+
+def _payload(gpu, o, g, scale, seed):
+    codes, scales, _, perm = config_codes(o, 128 * g, seed=seed, scale_dtype=DT[scale], permute=True)
+    zeros = torch.randint(0, 8, (g, o), generator=torch.Generator().manual_seed(seed), dtype=torch.uint8)
+    return {n: v.to(gpu) for n, v in layout_from_codes(codes, scales, zeros, perm).items()}
+
+
+@pytest.mark.parametrize("dtype,scale", [("bf16", "f16"), ("f16", "f16"), ("f16", "bf16")])
+@pytest.mark.parametrize("g,gps", [(5, 1), (6, 2), (8, 4), (11, 11), (33, 16)])
+def test_split_zero_points_of_eight_bits(gpu, g, gps, dtype, scale):
+    """Zero-points over the whole byte (the checked layouts hold 0..7): s (q - z) x has up
+    to 30 bits, and a product is off by its fp32 roundings alone: a single activation,
+    so that no sum hides them, within 2^-21 of the product (at most three additions of
+    its digits' products, an ulp each); and whole rows as above."""
+    layout = _payload(gpu, 37, g, scale, g)
+    wide = torch.randint(0, 256, (g, 37), generator=torch.Generator().manual_seed(1), dtype=torch.uint8).to(gpu)
+    some = torch.rand(g, 37, generator=torch.Generator().manual_seed(2)).to(gpu) < 0.3
+    layout["zeros"] = torch.where(some, wide, layout["zeros"])
+    decodeds = (False, True) if scale == "bf16" else (False,)
+    row = torch.randn(1, 128 * g, generator=torch.Generator().manual_seed(3)).to(DT[dtype]).to(gpu)
+    for decoded in decodeds:
+        want, terms = _expected(layout, row, gps, decoded)
+        assert bool(((_partials(layout, row, gps, decoded).double() - want).abs() <= 2.0 ** -18 * terms).all())
+        for column in range(0, 128 * g, 61):
+            x = torch.zeros_like(row)
+            x[0, column] = row[0, column]
+            want, _ = _expected(layout, x, gps, decoded)
+            assert bool(((_partials(layout, x, gps, decoded).double() - want).abs() <= 2.0 ** -21 * want.abs()).all())
+
+
+@pytest.mark.parametrize("decoded", [False, True])
+@pytest.mark.parametrize("g,gps", [(6, 1), (7, 2), (8, 4)])
+def test_split_scales_without_a_product(gpu, g, gps, decoded):
+    """A scale that is not finite stays in its own row and split (the other splits of its
+    four groups may be summed in another order); one so large that its products with a code
+    overflow still gives the sum that does not."""
+    layout = _payload(gpu, 40, g, "bf16", 3)
+    x = (torch.randn(1, 128 * g, generator=torch.Generator().manual_seed(3)) * 2.0 ** -20).to(torch.bfloat16).to(gpu)
+    clean = _partials(layout, x, gps, decoded)
+    layout["scales"][1, 3], layout["scales"][1, 20], layout["scales"][5, 39] = float("inf"), float("nan"), 3e38
+    got = _partials(layout, x, gps, decoded)
+    own, near = torch.zeros_like(got, dtype=torch.bool), torch.zeros_like(got, dtype=torch.bool)
+    for group, row in ((1, 3), (1, 20), (5, 39)):
+        own[group // gps, row] = True
+        near[[i // gps for i in range(group // 4 * 4, min(g, group // 4 * 4 + 4))], row] = True
+    assert torch.equal(got[~near], clean[~near])
+    want, terms = _expected(layout, x, gps, decoded)
+    near &= ~own
+    assert bool(((got[near].double() - want[near]).abs() <= 2.0 ** -18 * terms[near]).all())
+    assert not bool(torch.isfinite(got[1 // gps, 3])) and bool(torch.isnan(got[1 // gps, 20]))
+    want, terms = _expected(layout, x, gps, False)
+    if not decoded:  # (three times 3e38 has no bf16 value to round to)
+        assert bool(torch.isinf(got[1 // gps, 3]))
+        big = (5 // gps, 39)
+        assert bool((got[big].double() - want[big]).abs() <= 2.0 ** -18 * terms[big])
