@@ -333,6 +333,7 @@ __global__ __launch_bounds__(256) void head_norm_rope_kernel(HeadNormRopeArgs a)
       hi = rnd<DT>(to_f32<DT>(w[i + half]) * rnd<DT>(hi * inv));
     }
     if (rope) {
+#pragma clang fp contract(off)  // the roundings of rope_vector_kernel, which takes the longer sequences
       const float c0 = to_f32<DT>(cs[i]), c1 = to_f32<DT>(cs[i + half]);
       const float s0 = to_f32<DT>(sn[i]), s1 = to_f32<DT>(sn[i + half]);
       // rotate_half(y) = (-y[half:], y[:half])

@@ -56,22 +56,22 @@ def test_vector_rope_is_bit_exact(gpu, dtype, batch, hq, hk, seq, dim):
         # the algebra on the CPU (torch's GPU addcmul rounds rare fp16 sums differently)
         for a, b in zip(got, _rope_torch(*(v.cpu() for v in (*views, cos, sin)), axis)):
             assert torch.equal(a.cpu(), b)
-    if dtype == "f16":
-        return  # the row kernel's fp16 sum can round once where the algebra rounds to fp32 and then to fp16
     odd = normal(batch * seq * hq * dim + 1)[1:].view(batch, seq, hq, dim)  # off 16-byte alignment: the row kernel
-    for a, b in zip(fused_apply_rotary_pos_emb(odd, k, cos, sin, unsqueeze_dim=2), _rope_torch(odd, k, cos, sin, 2)):
-        assert torch.equal(a, b)
+    for a, b in zip(fused_apply_rotary_pos_emb(odd, k, cos, sin, unsqueeze_dim=2),
+                    _rope_torch(*(v.cpu() for v in (odd, k, cos, sin)), 2)):
+        assert torch.equal(a.cpu(), b)
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
 @pytest.mark.parametrize("mode", [_lib.ROPE_STOCK, _lib.ROPE_FUSED])
-def test_vector_rope_and_copy_into_a_cache(gpu, mode):
+def test_vector_rope_and_copy_into_a_cache(gpu, mode, dtype):
     """Rotation and a plain strided copy in one launch, each into its own slots, and the
     same bits as the row kernel (which a single position takes)."""
     heads, seq, dim, length = 6, 20, 128, 64
     g = torch.Generator().manual_seed(7)
-    x = torch.randn(2, seq, heads, dim, generator=g).to(torch.bfloat16).to(gpu)
-    cos, sin = (torch.randn(seq, dim, generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
-    cache = torch.full((2, heads, length, dim), 7.0, dtype=torch.bfloat16, device=gpu)
+    x = torch.randn(2, seq, heads, dim, generator=g).to(DT[dtype]).to(gpu)
+    cos, sin = (torch.randn(seq, dim, generator=g).to(DT[dtype]).to(gpu) for _ in range(2))
+    cache = torch.full((2, heads, length, dim), 7.0, dtype=DT[dtype], device=gpu)
     rows = torch.full_like(cache, 7.0)
 
     def tensors(dst, first, n):
