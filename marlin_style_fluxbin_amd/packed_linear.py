@@ -67,11 +67,11 @@ def holds_values(t: torch.Tensor, recording: bool) -> bool:
 
 def plain_call(x: torch.Tensor) -> bool:
     """True when a kernel called by address computes what a torch op on ``x`` would:
-    a plain tensor that holds its own values (no lazy negation), and no tracer, dispatch
-    or function mode, transform (vmap, jvp) or autocast in force that has to see (or
-    would change) the op."""
-    return (untraced() and type(x) is torch.Tensor and not x.is_neg() and not torch.is_autocast_enabled("cuda")
-            and torch._C._len_torch_function_stack() == 0 and untransformed())
+    a plain strided tensor that holds its own values (no lazy negation), and no tracer,
+    dispatch or function mode, transform (vmap, jvp) or autocast in force that has to see
+    (or would change) the op."""
+    return (untraced() and type(x) is torch.Tensor and x.layout is torch.strided and not x.is_neg()
+            and not torch.is_autocast_enabled("cuda") and torch._C._len_torch_function_stack() == 0 and untransformed())
 
 
 class PackedLinearBase(nn.Module):

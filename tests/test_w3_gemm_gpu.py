@@ -30,7 +30,10 @@ def _check(module, x, dtype):
     """The module's output within the bar of the exact product of its dense weight."""
     assert module._gemm_takes(x)
     with torch.inference_mode():
-        y = module(x)
+        _within(module, x, module(x), dtype)
+
+
+def _within(module, x, y, dtype):
     w = restore_planar_w3(module.layout(), dtype=x.dtype).double()
     flat = x.reshape(-1, module.in_features).double()
     exact = flat @ w.t()
@@ -133,3 +136,23 @@ def test_gemm_leaves_lazy_negation_to_torch(gpu):
     with torch.inference_mode():
         want = torch.nn.functional.linear(lazy, module._dense_weight(torch.float16))
         assert torch.equal(module(lazy), want)
+
+
+def test_gemm_leaves_sparse_inputs_to_torch(gpu):
+    """A sparse input has no memory to read by address: torch multiplies (or refuses) it."""
+    module = _module(gpu, 64, 256, scale="f16")
+    dense = torch.zeros(20, 256, device=gpu, dtype=torch.float16)
+    dense[3, 5], dense[7, 200] = 1.5, -2.0
+    for sparse in (dense.to_sparse(), dense.to_sparse_csr()):
+        assert not module._gemm_takes(sparse)
+
+        def outcome(call):
+            with torch.inference_mode():
+                try:
+                    return call()
+                except (RuntimeError, NotImplementedError) as error:
+                    return str(error)
+
+        want = outcome(lambda: torch.nn.functional.linear(sparse, module._dense_weight(torch.float16)))
+        got = outcome(lambda: module(sparse))
+        assert got == want if isinstance(want, str) else torch.equal(got, want)
