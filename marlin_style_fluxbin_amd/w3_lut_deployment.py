@@ -28,7 +28,7 @@ import torch
 from torch import nn
 
 from . import _lib
-from .packed_linear import HALF_DTYPES, PackedLinearBase, plain_call, replace_linears_atomically
+from .packed_linear import HALF_DTYPES, PackedLinearBase, holds_values, plain_call, replace_linears_atomically
 from .gptq_deployment import FIELDS, OPTIONAL_FIELDS, restore_planar_w3, validate_planar_w3
 
 ROW_TILES = (256, 512, 1024)
@@ -474,7 +474,7 @@ class PackedW3Linear(PackedLinearBase):
                 and 0 < x.numel() <= GEMM_MAX_ROWS * self.in_features
                 and planes.numel() < 2**31 and planes.data_ptr() % 16 == 0 and self._tensor("perm").data_ptr() % 16 == 0
                 and (bias is None or (bias.dtype == x.dtype and bias.device == x.device and bias.is_contiguous()
-                                      and bias.shape == (self.out_features,))))
+                                      and holds_values(bias, False) and bias.shape == (self.out_features,))))
 
     def _dense_linear(self, x: torch.Tensor) -> torch.Tensor:
         if self._gemm_takes(x):

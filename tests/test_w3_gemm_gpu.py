@@ -156,3 +156,13 @@ def test_gemm_leaves_sparse_inputs_to_torch(gpu):
         want = outcome(lambda: torch.nn.functional.linear(sparse, module._dense_weight(torch.float16)))
         got = outcome(lambda: module(sparse))
         assert got == want if isinstance(want, str) else torch.equal(got, want)
+
+
+def test_gemm_leaves_lazily_negated_biases_to_torch(gpu):
+    module = _module(gpu, 64, 256, bias=torch.zeros(64, device=gpu, dtype=torch.bfloat16))
+    module.bias = torch._neg_view(torch.ones(64, device=gpu, dtype=torch.bfloat16))
+    x = torch.randn(20, 256, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).to(gpu)
+    assert module.bias.is_neg() and not module._gemm_takes(x)
+    with torch.inference_mode():
+        want = torch.nn.functional.linear(x, module._dense_weight(torch.bfloat16), module.bias)
+        assert torch.equal(module(x), want)
