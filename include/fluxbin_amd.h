@@ -519,7 +519,8 @@ int fx_hybrid_gemv_segments_rmsnormed(const void *h, int x_dtype, int n_segments
  * [O, K] of a hybrid layout in weight_dtype (fp32, fp16 or bf16), 16-byte
  * aligned, bitwise the reference's fp32 arithmetic rounded once.  interleaved
  * != 0: codes [G, O, 32] and sparse_codes [G, O, 2] hold two bits a column
- * (base b of column i at bit 2 i + b), else the planes of fx_hybrid_gemv.  *bad
+ * (base b of column i at bit 2 i + b), else the planes of fx_hybrid_gemv.  The four
+ * scale arrays 8-byte aligned, both code arrays 2-byte aligned.  *bad
  * (device-accessible, cleared by the caller) becomes 1 when a scale is not
  * finite or a group's refinement indices are not ascending in [0, 128); the
  * weight then holds unspecified values in those groups.

@@ -1729,7 +1729,7 @@ int fx_hybrid_restore(const uint8_t* codes, const float* rows, const float* colu
   if (O < 1 || O > 65536) return fail(FX_EINVAL, "O must be in [1, 65536], got %d", O);
   if (K < 128 || K > 131072 || K % 128) return fail(FX_EINVAL, "K must be a multiple of 128 in [128, 131072]");
   if (reinterpret_cast<uintptr_t>(weight) % 16 != 0) return fail(FX_EINVAL, "weight must be 16-byte aligned");
-  const void* vec[3] = {rows, sparse_rows, columns};
+  const void* vec[4] = {rows, sparse_rows, columns, sparse_columns};
   for (const void* p : vec)
     if (reinterpret_cast<uintptr_t>(p) % 8 != 0) return fail(FX_EINVAL, "scales must be 8-byte aligned");
   if (reinterpret_cast<uintptr_t>(codes) % 2 != 0 || reinterpret_cast<uintptr_t>(sparse_codes) % 2 != 0)

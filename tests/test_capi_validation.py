@@ -296,6 +296,10 @@ CASES = [
     ("fx_hybrid_restore", dict(K=200), "K must be a multiple of 128 in [128, 131072]"),
     ("fx_hybrid_restore", dict(weight=D + 8), "weight must be 16-byte aligned"),
     ("fx_hybrid_restore", dict(rows=D + 4), "scales must be 8-byte aligned"),
+    ("fx_hybrid_restore", dict(sparse_rows=D + 4), "scales must be 8-byte aligned"),
+    ("fx_hybrid_restore", dict(columns=D + 4), "scales must be 8-byte aligned"),
+    ("fx_hybrid_restore", dict(sparse_columns=D + 4), "scales must be 8-byte aligned"),
+    ("fx_hybrid_restore", dict(sparse_codes=D + 1), "codes must be 2-byte aligned"),
     ("fx_hybrid_restore", dict(codes=D + 1), "codes must be 2-byte aligned"),
 ]
 
