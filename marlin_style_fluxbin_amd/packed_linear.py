@@ -29,34 +29,49 @@ import torch
 from torch import nn
 from torch.autograd import forward_ad
 from torch.nn import functional as F
-from torch.overrides import _get_current_function_mode_stack
-from torch.utils._device import DeviceContext
+
+try:
+    from torch.utils._device import DeviceContext
+except ImportError:  # then no function mode counts as the default device
+    DeviceContext = None
 
 HALF_DTYPES = (torch.float16, torch.bfloat16)
 PACKED_M1, DENSE_FALLBACK, PACKED_SMALL_M = "packed_m1", "dense_fallback", "packed_small_m"
 
 _PLAIN_TYPES = (torch.Tensor, nn.Parameter)
+
+
+def _query(owner, name: str, in_force):
+    """torch's own query ``name`` (they are internal and may be absent in another torch),
+    or one that always reports the state as in force: calls then keep the torch ops."""
+    return getattr(owner, name, None) or (lambda: in_force)
+
+
+_dispatch_modes = _query(torch._C, "_len_torch_dispatch_stack", 1)
+_function_modes = _query(torch._C, "_len_torch_function_stack", 1)
+_function_mode_stack = _query(torch.overrides, "_get_current_function_mode_stack", (None,))
+_tracer = _query(torch._C, "_get_tracing_state", True)
+_transform_level = _query(getattr(torch._C, "_functorch", None), "maybe_current_level", 0)
+
 PackedKernel = Callable[[torch.Tensor, torch.Tensor], torch.Tensor]  # (x [rows, K], out [rows, O]) -> out
 
 
 def untraced() -> bool:
     """True when no tracer or dispatch mode records the torch ops of this call: what a
     kernel called by address writes would be missing from such a record."""
-    return (not torch.compiler.is_compiling() and torch._C._len_torch_dispatch_stack() == 0
-            and torch._C._get_tracing_state() is None)
+    return not torch.compiler.is_compiling() and _dispatch_modes() == 0 and _tracer() is None
 
 
 def untransformed() -> bool:
     """True when no transform (vmap, jvp, grad) and no forward-mode level is in force: what
     a kernel called by address writes carries neither a batch dimension nor a tangent."""
-    return torch._C._functorch.maybe_current_level() is None and forward_ad._current_level < 0
+    return _transform_level() is None and getattr(forward_ad, "_current_level", 0) < 0
 
 
 def only_default_device() -> bool:
     """True when no torch function mode but torch's own default-device context (which
     changes factory calls alone) is in force."""
-    return torch._C._len_torch_function_stack() == 0 or all(
-        type(mode) is DeviceContext for mode in _get_current_function_mode_stack())
+    return _function_modes() == 0 or all(type(mode) is DeviceContext for mode in _function_mode_stack())
 
 
 def holds_values(t: torch.Tensor, recording: bool) -> bool:
@@ -71,7 +86,7 @@ def plain_call(x: torch.Tensor) -> bool:
     dispatch or function mode, transform (vmap, jvp) or autocast in force that has to see
     (or would change) the op."""
     return (untraced() and type(x) is torch.Tensor and x.layout is torch.strided and not x.is_neg()
-            and not torch.is_autocast_enabled("cuda") and torch._C._len_torch_function_stack() == 0 and untransformed())
+            and not torch.is_autocast_enabled("cuda") and _function_modes() == 0 and untransformed())
 
 
 class PackedLinearBase(nn.Module):

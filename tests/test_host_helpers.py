@@ -2,13 +2,15 @@
 quantizer (config 3's weights), the rank-one layout contract, the tensor hash,
 the Qwen3-8B shape table and the GPU-only guards of the HIP entry points."""
 import hashlib
+import importlib.util
 import json
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
 import torch
 
-from marlin_style_fluxbin_amd import _lib
+from marlin_style_fluxbin_amd import _lib, packed_linear
 from marlin_style_fluxbin_amd.deployment import load_extension
 from marlin_style_fluxbin_amd.evaluation import tensor_sha256
 from marlin_style_fluxbin_amd.qwen3 import qwen3_8b_linear_shapes, quantize_w3_rtn
@@ -115,3 +117,46 @@ def test_gpu_only_guards():
     if not torch.cuda.is_available():
         with pytest.raises(RuntimeError, match="no CPU substitute"):
             load_extension("v1")
+
+
+_QUERIES = [("_C", "_len_torch_dispatch_stack"), ("_C", "_len_torch_function_stack"), ("_C", "_get_tracing_state"),
+            ("_C", "_functorch"), ("autograd.forward_ad", "_current_level")]
+
+
+@pytest.mark.parametrize("owner,name", _QUERIES)
+def test_a_torch_without_an_internal_query_keeps_the_torch_ops(monkeypatch, owner, name):
+    """The gates of the kernels called by address ask torch's internals; one that is
+    missing counts as a state in force and raises nothing."""
+    x = torch.ones(2, 128)
+    assert packed_linear.plain_call(x)
+    module = torch
+    for part in owner.split("."):
+        module = getattr(module, part)
+    monkeypatch.delattr(module, name)
+    spec = importlib.util.spec_from_file_location("packed_linear_elsewhere", packed_linear.__file__)
+    elsewhere = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(elsewhere)
+    assert not elsewhere.plain_call(x)
+
+
+def test_gates_see_modes_transforms_and_graphs():
+    with torch.device("cpu"):  # torch's default device is a function mode that changes factory calls alone
+        assert packed_linear.only_default_device() and not packed_linear.plain_call(torch.ones(2))
+    with torch.overrides.BaseTorchFunctionMode():
+        assert not packed_linear.only_default_device()
+    leaf = torch.ones(2, requires_grad=True)
+    assert not packed_linear.holds_values(leaf, True) and packed_linear.holds_values(leaf, False)
+    assert not packed_linear.holds_values(torch._neg_view(torch.ones(2)), False)
+    seen = []
+    torch.func.vmap(lambda x: (seen.append(packed_linear.untransformed()), x)[1])(torch.ones(2, 2))
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(packed_linear.untransformed())
+    assert seen == [False, False] and packed_linear.untransformed()
+    assert not packed_linear.plain_call(torch.ones(2, 2).to_sparse())
+
+
+def test_stream_handle_without_the_raw_query(monkeypatch):
+    monkeypatch.setattr(_lib, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: SimpleNamespace(cuda_stream=(77, device)))
+    assert _lib.stream_handle() == (77, None)
+    assert _lib.stream_handle(torch.device("cuda", 1)) == (77, torch.device("cuda", 1))
