@@ -166,3 +166,14 @@ def test_gemm_leaves_lazily_negated_biases_to_torch(gpu):
     with torch.inference_mode():
         want = torch.nn.functional.linear(x, module._dense_weight(torch.bfloat16), module.bias)
         assert torch.equal(module(x), want)
+
+
+# more rows than the module's route takes, as a caller of the C entry may pass: plans of
+# both kernels, whole and ragged sizes, one and two K splits, and the last row allowed
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("m,o,k", [(513, 17, 256), (513, 200, 8192), (700, 12300, 384), (1500, 330, 1408), (1500, 3000, 640),
+                                   (4097, 65, 128), (8192, 200, 640), (8192, 1001, 384)])
+def test_gemm_entry_beyond_the_modules_rows(gpu, m, o, k, dtype):
+    module = _module(gpu, o, k, seed=m, permute=m % 2 == 1)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(DT[dtype]).to(gpu)
+    _within(module, x, module._gemm(x, m), dtype)

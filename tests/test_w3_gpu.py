@@ -128,6 +128,73 @@ def test_reference_split_contract(gpu, row_tile, dtype):
                 assert_rel(corrected.float().cpu().numpy(), decoded, HALF_TOL)
 
 
+# The table kernel (w3_lut.hip) serves what the one-row matrix-core kernel does not: splits
+# of 3, 5, 6, 7 ... groups, K > 16384, and several rows.
+#
+# Bar: a product passes through at most 128 fp32 additions (7 in its table, 48 and 19 in
+# its group, one per group of a split, one per split), each off by at most 2^-24 of the
+# unsigned terms' sum (q <= 7, z <= 4: at most 11 s |x| a column): 2^-17 of that sum.
+def _split_truth(layout, ol, x, gps, decoded):
+    """float64 partials [splits, M, O] and 2^-17 of each one's terms."""
+    d = w3.signed_codes_sorted(ol).astype(np.float64)
+    s = np.repeat(np.asarray(ol["scales"], dtype=np.float64).T, 128, axis=1)
+    w = torch.from_numpy(s * d)
+    if decoded:
+        w = w.to(torch.bfloat16).double()
+    xs = x.double()[:, layout["perm"].long()]
+    step, k = 128 * gps, x.shape[1]
+    parts = torch.stack([xs[:, i:i + step] @ w[:, i:i + step].t() for i in range(0, k, step)])
+    terms = torch.stack([xs[:, i:i + step].abs() @ torch.from_numpy(s)[:, i:i + step].t() for i in range(0, k, step)])
+    return parts, 2.0 ** -17 * 11 * terms
+
+
+def _assert_split(out, ws, parts, slack):
+    """The workspace within the bar of every partial, the output within it and half an ulp."""
+    if ws is not None:
+        assert bool(((ws.cpu().double().reshape(parts.shape) - parts).abs() <= slack).all())
+    exact, total = parts.sum(0), slack.sum(0)
+    bits, low = (7, -126) if out.dtype == torch.bfloat16 else (10, -14)
+    ulp = torch.exp2(torch.floor(torch.log2(exact.abs().clamp(min=2.0 ** low))) - bits)
+    assert bool(((out.cpu().double() - exact).abs() <= 0.5 * ulp + total).all())
+
+
+@pytest.mark.parametrize("row_tile", [256, 512, 1024])
+@pytest.mark.parametrize("o,k,gps", [(1, 512, 3), (300, 896, 3), (1030, 1280, 5), (65, 896, 6), (257, 1024, 7),
+                                     (40, 16512, 4), (33, 16512, 1)])
+def test_table_kernel_splits(gpu, row_tile, o, k, gps):
+    """One row: the partials of every split and the output, both arithmetics, on a
+    poisoned workspace."""
+    layout, dl, ol = _setup(o, k, seed=o + gps, permute=True)
+    for dtype in (torch.bfloat16, torch.float16):
+        x = _x(1, k, dtype, seed=gps)
+        for arithmetic in ("structural", "decoded_bf16"):
+            ws = torch.full(workspace_shape(o, k, gps), float("nan"), device=gpu)
+            out = torch.empty(1, o, dtype=dtype, device=gpu)
+            w3_lut_m1_out(x.to(gpu), dl, out, ws, row_tile=row_tile, groups_per_split=gps, arithmetic=arithmetic)
+            _assert_split(out, ws, *_split_truth(layout, ol, x, gps, arithmetic == "decoded_bf16"))
+
+
+@pytest.mark.parametrize("arithmetic", ["structural", "decoded_bf16"])
+@pytest.mark.parametrize("m", [2, 4, 8])
+@pytest.mark.parametrize("o,k,gps", [(65, 512, 4), (300, 896, 2), (257, 1280, 3)])
+def test_table_kernel_rows(gpu, m, o, k, gps, arithmetic):
+    """Several rows, whole and split K, and the eager route of decoded_bf16 (3 rows as
+    blocks of 2 and 1)."""
+    layout, dl, ol = _setup(o, k, seed=m + o, permute=True)
+    x = _x(m, k, torch.bfloat16, seed=m)
+    splits = workspace_shape(o, k, gps)[0]
+    ws = torch.full((splits, m, o), float("nan"), device=gpu)
+    out = torch.empty(m, o, dtype=torch.bfloat16, device=gpu)
+    w3_lut_m1_out(x.to(gpu), dl, out, ws, row_tile=512, groups_per_split=gps, arithmetic=arithmetic)
+    decoded = arithmetic == "decoded_bf16"
+    _assert_split(out, ws if splits > 1 else None, *_split_truth(layout, ol, x, gps, decoded))
+    for rows in {3, m} if decoded else ():
+        x = _x(rows, k, torch.bfloat16, seed=rows)
+        out = torch.empty(rows, o, dtype=torch.bfloat16, device=gpu)
+        W3Gemv(dl, arithmetic=arithmetic, max_rows=8)(x.to(gpu), out)
+        _assert_split(out, None, *_split_truth(layout, ol, x, gps, True))
+
+
 def test_fused_path_graph_replays_track_input(gpu):
     """Graph-captured single-launch GEMV: every replay equals the eager result for
     the current input (the in-launch split counters must reset every time)."""
