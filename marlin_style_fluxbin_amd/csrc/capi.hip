@@ -1184,11 +1184,12 @@ int fx_w3_restore(const uint8_t* planes, const void* scales, int scale_dtype,
 
 namespace {
 
-// Tiling of the W3 GEMM.  The activation tile is the smallest that holds the rows
-// (past 112 rows, 7 or 8 tiles of 16, whichever pads less).  Its wide form (3 or 4
-// output tiles a workgroup: each activation operand feeds that many) runs where it
-// gives three quarters of the CUs a workgroup; else the narrow form, one tile (two
-// with 64 rows and more, or where K is split: twice the rows per operand).  K is
+// Tiling of the W3 GEMM.  Up to 64 rows the activation tile is the smallest multiple of 16
+// that holds them; above, 7 or 8 tiles of 16, whichever pads less (65..112 rows: 7).  The
+// wide form (3 output tiles a workgroup, 4 above 64 rows: each activation operand feeds
+// that many) runs where it gives three quarters of the CUs a workgroup; else the narrow
+// form, one output tile (two from 49 rows on, or where K has 16 batches of 512 columns:
+// twice the rows per operand).  K is
 // split over workgroups only where the grid leaves half of the CUs without one and
 // every wave still has a batch: the splits' fp32 partials cost a finish launch.
 // Measured (bf16, us a launch, 40 rotating payloads in a graph; 37 rows): 12288 x

@@ -22,7 +22,7 @@
 // [O, K] tensors and four host synchronisations each) and takes 0.47 ms with this
 // kernel and one wait, bound by the host (this kernel 148 us of it, the products 162; a
 // check launch of its own, so that the host waits less, gained nothing).  The seven
-// launches' mean is 21.1 us (32.5 with the refined columns selected in registers).
+// launches' mean is 21.3 us (32.5 with the refined columns selected in registers).
 #include "common.h"
 #include "two_base_launch.h"
 

@@ -22,11 +22,12 @@
 // Step (w, b) of a batch multiplies columns 32 w + 8 b .. + 7 of each group.
 //
 // Work split: a workgroup owns 16 RT output rows, 16 MT activation rows and a K
-// range whose batches its NK waves take in turn; their sums meet in LDS, pairwise.  No two waves of a workgroup read the same weights or activations, so
-// nothing is staged: gemm_pack_kernel has laid the activations out in operand order
-// (and in the payload's column order) once, and every B operand is one coalesced
-// 16-byte load per lane, issued PD half-words (two steps each) ahead.  K splits over
-// workgroups leave fp32 partials for gemm_finish_kernel, in split order.
+// range whose batches its NK waves take in turn; their sums meet in LDS, pairwise.  No
+// two waves of a workgroup read the same weights or activations, so nothing is staged:
+// gemm_pack_kernel has laid the activations out in operand order (and in the payload's
+// column order) once, and every B operand is one coalesced 16-byte load per lane, issued
+// PD half-words (two steps each) ahead.  K splits over workgroups leave fp32 partials
+// for gemm_finish_kernel, in split order.
 #pragma once
 #include "w3_gemm_launch.h"
 #include "w3_mfma.hip"

@@ -6,7 +6,7 @@
 // row and group, which serialise on banks, and a second launch summed its partials.
 // Here a (row, group)'s eight weight values become matrix operands by byte lookup
 // (w3_values.h), about two VALU instructions a weight.  Measured (bf16, desc_act,
-// decoded_bf16): 12288 x 4096 in 8 splits 10.6 us and 4096 x 12288 in 48 splits 11.4 us
+// decoded_bf16): 12288 x 4096 in 8 splits 10.9 us and 4096 x 12288 in 48 splits 11.4 us
 // a launch (two layers' Linears on the observed_exact route, six of these and eight
 // one-split launches: 315 -> 110 us).  The bound is the chain of loads, gather and
 // expansion of six waves a SIMD (with 92 registers, five waves: 11.2).

@@ -84,7 +84,7 @@ def plain_call(x: torch.Tensor) -> bool:
     """True when a kernel called by address computes what a torch op on ``x`` would:
     a plain strided tensor that holds its own values (no lazy negation), and no tracer,
     dispatch or function mode, transform (vmap, jvp) or autocast in force that has to see
-    (or would change) the op."""
+    (or would change) the op.  (A default device, which is a function mode, counts.)"""
     return (untraced() and type(x) is torch.Tensor and x.layout is torch.strided and not x.is_neg()
             and not torch.is_autocast_enabled("cuda") and _function_modes() == 0 and untransformed())
 

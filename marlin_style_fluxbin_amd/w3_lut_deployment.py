@@ -35,10 +35,12 @@ ROW_TILES = (256, 512, 1024)
 EXPERIMENTAL_ROW_TILES = ROW_TILES
 ARITHMETIC_MODES = ("structural", "decoded_bf16")
 MAX_PACKED_ROWS = 8
-# Dense-fallback rows that fx_w3_gemm multiplies.  Above them the restored weight's
-# library product is as fast or faster (measured, us, GEMM / restore + product, identity
-# order: 512 rows 12288 x 4096 62.6 / 77.7, 4096 x 4096 31.1 / 37.7, 4096 x 12288 68.5 /
-# 95.3; 640 rows 102 / 86, 52 / 42, 89 / 108; 1024 rows 116 / 110, 53 / 48, 125 / 127).
+# Dense-fallback rows that fx_w3_gemm multiplies, one limit for every shape and column
+# order.  Measured (us, GEMM / restore + library product, identity order): 512 rows 12288 x
+# 4096 62.6 / 77.7, 4096 x 4096 31.1 / 37.7, 4096 x 12288 68.5 / 95.3; 640 rows 102 / 86,
+# 52 / 42, 89 / 108; 1024 rows 116 / 110, 53 / 48, 125 / 127.  So above the limit the library
+# wins at K = 4096 and the GEMM still leads at 4096 x 12288; with a column permutation the
+# restore costs 28-44 % more, which moves the crossing up further.
 GEMM_MAX_ROWS = 512
 QWEN3_ROW_TILE_BY_SHAPE = {
     (4096, 4096): 256,

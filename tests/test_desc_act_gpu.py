@@ -162,7 +162,7 @@ def test_native_session_table_routes(gpu, route):
     """Table-route Linears (decoded_bf16 arithmetic; observed_exact also two groups
     per split) run their own split contract in the native decode: every Linear's
     decode call bit-equals the module's forward, and the session matches HF with
-    the same modules.  desc_act payloads, so the table kernel's gather runs too."""
+    the same modules.  desc_act payloads, so the split kernel's gather runs too."""
     print(f"native decode, table route {route}", flush=True)
     model, ids, forced = _small(gpu, desc_act_seed=3, scale_dtype=torch.bfloat16, zeros=False)
     gps = 2 if route == "observed_exact" else 1

@@ -5,8 +5,8 @@ The fixtures are frozen outputs of the CPU oracle (``tests/golden/make_golden.py
 path runs on the payloads stored in them:
 
 * W3 GEMV at the reference's own test shapes (64 x 256, 288 x 384; the reference's
-  GPTQ generator, desc_act permutation): the MFMA fast path and the table kernel
-  of the reference contract, bf16 and fp16 activations, within half an output ulp
+  GPTQ generator, desc_act permutation): the MFMA fast path and the reference's
+  split contract (one row: the matrix-core split kernel), bf16 and fp16 activations, within half an output ulp
   of the float64 structural truth; the decoded-bf16 arithmetic against the
   float64 dequantize-then-matmul; the restore kernel bit for bit (sha256);
 * config 0 (q_proj 4096 x 4096, fp16 scales, zero-points U{3,4}): payload bytes
@@ -67,7 +67,7 @@ def test_w3_gemv_golden(gpu, name):
                 y = torch.empty(1, o, dtype=dtype, device=gpu)
                 w3_lut_m1_out(x, layout, y, ws, row_tile=row_tile, groups_per_split=gps)
                 assert_half_ulp(y.float().cpu().numpy(), f[exact_key], label, rel_slack=2e-6,
-                                what=f"{name} table path {label} rt {row_tile} gps {gps}")
+                                what=f"{name} split contract {label} rt {row_tile} gps {gps}")
     xb = _bits_to(f["x_bf16_bits"], torch.bfloat16, gpu).reshape(1, k)
     fp32 = gemv_fp32_device(xb, layout, arithmetic="structural").cpu().numpy()
     exact = f["y_exact_bf16x"]

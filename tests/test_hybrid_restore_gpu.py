@@ -1,6 +1,7 @@
 """``fx_hybrid_restore`` (the hybrid Linear's dense fallback) against the torch
 arithmetic it replaces on the GPU: bitwise in every output type and both code
-formats at row counts off the workgroup's 128 and 16, and the same refusals."""
+formats at row counts off a workgroup's 64 and a wave's 8, the same refusals, and the
+calls that keep the torch arithmetic."""
 import pytest
 import torch
 from torch.autograd import forward_ad

@@ -85,7 +85,9 @@ def test_fused_fast_path(gpu, o, k, m, xdtype, scale_dtype):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_reference_split_contract(gpu, row_tile, dtype):
     """Reference tests/test_w3_lut_correctness.py:51-135: NaN-poisoned workspace,
-    repeat-exact after re-poisoning, graph replay bit-equality, both arithmetics."""
+    repeat-exact after re-poisoning, graph replay bit-equality, both arithmetics.
+    One row and these splits run the matrix-core split kernel, for which the row tile is a
+    checked hint; the table kernel's own calls are below."""
     for out_features, in_features in ((32, 128), (64, 256), (288, 384)):
         layout, dl, ol = _setup(out_features, in_features, seed=out_features, zeros=False)
         x = _x(1, in_features, dtype, seed=in_features).to(gpu)

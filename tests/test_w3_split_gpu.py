@@ -1,7 +1,8 @@
 """The split contract's matrix-core kernel (``fx_w3_inline_main`` / ``fx_w3_m1_out``, one
 row) against float64 partial sums of the definition: every split form it takes, ragged
 sizes, both arithmetics, zero-points beyond 3 and 4 (where decoded_bf16 rounds only the
-weights with |q - z| = 3, as the table kernel does) and unaligned operands.
+weights with |q - z| = 3, as the table kernel does) and beyond 7, scales that no finite
+product has, and unaligned operands.
 
 Bar: every product is exact, so a partial is off by its fp32 additions alone: at most 32
 matrix instructions a batch (two chains of 16) and one addition a batch, each at most
