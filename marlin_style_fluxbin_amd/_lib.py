@@ -127,16 +127,18 @@ def ptr(tensor: torch.Tensor | None) -> int | None:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # internal: may be absent in another torch
+_GPU_INDEX = {torch.device("cuda", i): i for i in range(64)}
 
 
 def stream_handle(device: torch.device | None = None) -> int:
     """The current stream of ``device`` (default: the current device) as an integer,
     without building a ``torch.cuda.Stream`` for it (2.6 us of every call) where torch
-    offers that."""
-    if _raw_stream is None:
+    offers that.  Any other device is refused (by torch), so a call whose tensors are not
+    on a GPU ends before their addresses reach a kernel."""
+    index = _GPU_INDEX.get(device)
+    if index is None or _raw_stream is None:
         return torch.cuda.current_stream(device).cuda_stream
-    index = None if device is None else device.index
-    return _raw_stream(torch.cuda.current_device() if index is None else index)
+    return _raw_stream(index)
 
 
 def require_gpu_tensor(tensor: torch.Tensor, name: str) -> None:

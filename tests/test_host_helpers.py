@@ -160,3 +160,24 @@ def test_stream_handle_without_the_raw_query(monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: SimpleNamespace(cuda_stream=(77, device)))
     assert _lib.stream_handle() == (77, None)
     assert _lib.stream_handle(torch.device("cuda", 1)) == (77, torch.device("cuda", 1))
+
+
+@pytest.mark.parametrize("device", ["cpu", "meta", "cuda", None])
+def test_only_an_indexed_gpu_takes_the_raw_stream(monkeypatch, device):
+    """Every entry point asks for its stream before the C call: the query refuses tensors
+    that are on no GPU (torch's ValueError), and so their addresses reach no kernel."""
+    def current_stream(device=None):
+        if device is not None and device.type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {device}")
+        return SimpleNamespace(cuda_stream=5)
+
+    monkeypatch.setattr(torch.cuda, "current_stream", current_stream)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(_lib, "_raw_stream", lambda index: 100 + index)
+    assert _lib.stream_handle(torch.device("cuda", 3)) == 103
+    device = device if device is None else torch.device(device)
+    if device is None or device.type == "cuda":
+        assert _lib.stream_handle(device) in (5, 100)
+    else:
+        with pytest.raises(ValueError, match="Expected a cuda device"):
+            _lib.stream_handle(device)

@@ -17,6 +17,7 @@ from marlin_style_fluxbin_amd import (
     PackedW3Linear, W3Gemv, bf16_weight_semantics_w3_matvec, restore_planar_w3, structural_w3_matvec,
     w3_lut_m1_out, workspace_shape,
 )
+from marlin_style_fluxbin_amd import w3_lut_deployment as wl
 from oracle import w3
 from tests.payloads import assert_half_ulp, assert_rel, config_codes, layout_from_codes, oracle_layout
 
@@ -419,3 +420,15 @@ def test_engine_w3_backend_apply_out(gpu):
         W3Gemv(dl)(x, want)
         assert torch.equal(out.view(torch.int16), want.view(torch.int16))
     assert_half_ulp(out.float().cpu().numpy(), w3.matvec_exact(x.float().cpu().numpy(), ol), "bf16")
+
+
+def test_tensors_off_the_gpu_are_refused(gpu):
+    """A tensor in host memory ends in a ValueError before its address reaches a kernel."""
+    layout, dl, _ = _setup(64, 256, seed=1)
+    x, out = _x(1, 256, torch.bfloat16), torch.empty(1, 64, dtype=torch.bfloat16, device=gpu)
+    with pytest.raises(ValueError, match="cuda device"):
+        W3Gemv(dl)(x, out)
+    with pytest.raises(ValueError, match="cuda device"):
+        wl.finish(torch.zeros(2, 64), torch.empty(1, 64, dtype=torch.bfloat16), row_tile=256)
+    with pytest.raises(ValueError):
+        w3_lut_m1_out(x, dl, out, torch.empty(2, 64, device=gpu), row_tile=256)
